@@ -711,8 +711,8 @@ int tgs_rasterizer_backward_ex(tgs_rasterizer* r, const void* grad_image, const 
     hipStream_t s = (hipStream_t)stream;
     const int64_t n = r->n;
     TGS_TRY(ensure(r->grad2d, sizeof(float) * kGradStride * (size_t)(n > 0 ? n : 1), s));
-    TGS_TRY(ensure(r->heavy, sizeof(uint4) * (size_t)(n > 0 ? n : 1), s));
-    TGS_TRY(ensure(r->live, sizeof(uint4) * (size_t)(n > 0 ? n : 1), s));
+    TGS_TRY(ensure(r->heavy, sizeof(uint4) * (size_t)std::max<int64_t>(pb_list_entries(n), 1), s));
+    TGS_TRY(ensure(r->live, sizeof(uint4) * (size_t)std::max<int64_t>(pb_list_entries(n), 1), s));
     if (flags & ~(TGS_BACKWARD_ASSIGN | TGS_BACKWARD_SPARSE | TGS_BACKWARD_POSE | TGS_BACKWARD_KEEP_2D))
         return fail(TGS_ERR_INVALID, "unknown backward flags 0x%x", flags);
     if ((flags & TGS_BACKWARD_ASSIGN) && (flags & TGS_BACKWARD_SPARSE))

@@ -269,9 +269,11 @@ void launch_blend_backward(const CamParams& cam, const uint32_t* inst_vals, cons
 // mode: 0 accumulate, 1 assign, 2 sparse (assign rows with gradient, write
 // row_mask[i] = 1 for them and 0 for the others, leave the others untouched).
 enum { kGradAccumulate = 0, kGradAssign = 1, kGradSparse = 2 };
-// Scratch: live and heavy (n uint4 each) lists of the primitives with
+// Scratch: live and heavy (pb_list_entries(n) uint4 each) lists of the primitives with
 // records, grad2d (12 n floats).
 int64_t pb_chunks(int64_t n);
+// Entries of its live and heavy lists (whole chunks).
+int64_t pb_list_entries(int64_t n);
 // Records are counted by rec_count (cleared here for the next backward) and
 // on fp32 images marked by rec_mask (cleared here) and rec_bits.
 // slot_limit: the instance capacity of the forward (records lie below it).

@@ -365,6 +365,10 @@ constexpr int kClassChunk = 256 * kClassRounds;
 
 int64_t pb_chunks(int64_t n) { return n > 0 ? (n + kClassChunk - 1) / kClassChunk : 0; }
 
+// A chunk's slice starts at kClassChunk c and its primitives come from units
+// over the whole index range, so the last slice may reach past n.
+int64_t pb_list_entries(int64_t n) { return pb_chunks(n) * kClassChunk; }
+
 // Zeroes dst[0, n) with the lanes of one wave.
 __device__ __forceinline__ void zero_run(float* __restrict__ dst, int64_t n) {
     // the arrays are 16-byte aligned and a run starts at a multiple of 64
