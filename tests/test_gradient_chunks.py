@@ -7,7 +7,8 @@ import pytest
 
 from tinygs_amd import _lib
 
-SIZES = [1, 63, 64, 65, 255, 256, 257, 1023, 1024, 1025, 1100, 2047, 2049, 4097, 131071, 131073, 262145, 1_000_003]
+SIZES = [1, 63, 64, 65, 255, 256, 257, 1023, 1024, 1025, 1100, 2047, 2049, 4097, 131071, 131073, 262145, 524288, 524289, 525000,
+         1_000_003]
 
 
 def _fn(name):

@@ -27,6 +27,8 @@
 // zero, so their parameters are never read (at 1M Gaussians most visible
 // primitives sit behind others and fall in this class). SH-rest parameter
 // rows are read per thread, and only for primitives with gradients.
+#include <type_traits>
+
 #include "common.h"
 #include "halfmath.h"
 #include "kernels.h"
@@ -336,13 +338,13 @@ __device__ __forceinline__ void hs_result(const HalfSums& h, float4& gA, float4&
     gC = make_float4(hs_value(h, 8), hs_value(h, 9), (float)h.op, 0.f);
 }
 
-// One workgroup per chunk of 2048 primitives runs three phases (one launch;
-// the chunk's lists and heavy sums never leave the workgroup's own slices, so
-// the phases only need workgroup barriers). Chunk c holds the 64-primitive
-// units c, c + C, ..., c + 15 C (C chunks), one wave per unit and round:
-// spread over the whole index range, so every chunk gets a similar share of
-// the primitives that received a gradient even when the index order is
-// spatial (after Morton reordering the visible primitives are a few
+// One workgroup per chunk of primitives (256 per round, see pb_rounds) runs
+// three phases (one launch; the chunk's lists and heavy sums never leave the
+// workgroup's own slices, so the phases only need workgroup barriers). Chunk
+// c holds the 64-primitive units c, c + C, ... (C chunks), one wave per unit
+// and round: spread over the whole index range, so every chunk gets a similar
+// share of the primitives that received a gradient even when the index order
+// is spatial (after Morton reordering the visible primitives are a few
 // contiguous index runs: contiguous chunks of 2048 took 0.05 -> 0.51 ms).
 //
 // ---- phase 1: classify every primitive, list the live ones
@@ -360,14 +362,24 @@ __device__ __forceinline__ void hs_result(const HalfSums& h, float4& gA, float4&
 // (index, min(count, kLightRecords + 1) | span << 5, first slot, mask word of
 // ranks 0..31) and heavy (index, first slot + span, first slot, mask word);
 // fp16 images (index, count, first slot, 0) in both lists.
-constexpr int kClassRounds = 4;
-constexpr int kClassChunk = 256 * kClassRounds;
+constexpr int kManyRounds = 4;
+// Rounds of 256 primitives per chunk. A chunk is a chain of dependent loads
+// whatever its size, so up to 2,048 chunks of 256 (2^19 primitives) more
+// workgroups in flight win; beyond that the chip is full anyway and a chunk
+// of 1,024 fills phase 3's waves better where few primitives are live. One
+// round against four: 8.6 / 28 us at 1,024 primitives, 24 / 49 at 100k,
+// 37 / 46 at 201k, 63 / 75 at 500k; at 1M (8 % live) 76 / 57.
+constexpr int64_t kOneRoundMax = 1 << 19;
+static int pb_rounds(int64_t n) { return n <= kOneRoundMax ? 1 : kManyRounds; }
 
-int64_t pb_chunks(int64_t n) { return n > 0 ? (n + kClassChunk - 1) / kClassChunk : 0; }
+int64_t pb_chunks(int64_t n) {
+    const int64_t chunk = 256 * (int64_t)pb_rounds(n);
+    return n > 0 ? (n + chunk - 1) / chunk : 0;
+}
 
-// A chunk's slice starts at kClassChunk c and its primitives come from units
-// over the whole index range, so the last slice may reach past n.
-int64_t pb_list_entries(int64_t n) { return pb_chunks(n) * kClassChunk; }
+// A chunk's slice starts at the chunk size times c and its primitives come
+// from units over the whole index range, so the last slice may reach past n.
+int64_t pb_list_entries(int64_t n) { return pb_chunks(n) * 256 * pb_rounds(n); }
 
 // Zeroes dst[0, n) with the lanes of one wave.
 __device__ __forceinline__ void zero_run(float* __restrict__ dst, int64_t n) {
@@ -378,7 +390,7 @@ __device__ __forceinline__ void zero_run(float* __restrict__ dst, int64_t n) {
     for (int64_t e = (nv << 2) + lane; e < n; e += 64) dst[e] = 0.f;
 }
 
-template <bool kHalf>
+template <bool kHalf, int kClassRounds>
 __device__ __forceinline__ void classify_chunk(int64_t n, const uint32_t* __restrict__ rec_count,
                                                const uint32_t* __restrict__ rec_mask,
                                                const uint32_t* __restrict__ first_slot, const uint32_t* n_touched,
@@ -387,6 +399,7 @@ __device__ __forceinline__ void classify_chunk(int64_t n, const uint32_t* __rest
                                                uint4* __restrict__ heavy, uint32_t slot_limit, uint32_t* s_rw,
                                                uint32_t& n_live,
                                                uint32_t& n_heavy) {
+    constexpr int kClassChunk = 256 * kClassRounds;
     const uint32_t t = threadIdx.x;
     const int64_t c0 = (int64_t)blockIdx.x * kClassChunk;   // the chunk's slice of the lists
     // round r, wave v: unit blockIdx.x + (4 r + v) gridDim.x of 64 primitives
@@ -688,48 +701,68 @@ __device__ __forceinline__ void gather_heavy_chunk(const uint4* __restrict__ lis
 // Light primitives sum their (at most kLightRecords) records here, heavy ones
 // read grad2d. The record counter is cleared for the next backward. Rows are
 // scattered (live primitives are sparse), so every row access is one request
-// per lane: the 90-byte fp16 SH-rest row is read as 8-byte pieces of its
-// 8-byte-aligned window, realigned through the thread's LDS slot, and the
-// 180-byte SH-rest gradient row is written as 8-byte pairs (which pairs
-// depends on the row's 8-byte phase). Assign / sparse store the rows,
+// per lane: the 90-byte fp16 SH-rest row is read as 16-byte pieces of its
+// 4-byte-aligned window and realigned in registers, the fp32 row and the
+// 180-byte SH-rest gradient row move as 16-byte pieces at 4-byte boundaries. Assign / sparse store the rows,
 // accumulate adds to them; the SH-rest gradient row gets k_b * dL/dcolour_c
 // for the active bases b (kernels_backward.cuh:41-65) and, when stored,
 // zero for the others.
-constexpr int kShWin = 13;   // 8-byte words per LDS slot (an odd word stride)
+// 16 bytes at any 4-byte boundary: one request per lane and 4 floats
+typedef float v4f __attribute__((ext_vector_type(4)));
+typedef v4f v4f_any __attribute__((aligned(4)));
+typedef uint32_t v4u __attribute__((ext_vector_type(4)));
+typedef v4u v4u_any __attribute__((aligned(4)));
 
-template <typename ShT>
-__device__ __forceinline__ void load_sh_row(const ShT* __restrict__ shr_all, int64_t ip, int nsh, uint2* slot,
-                                            float shv[45]) {
-    const ShT* sr = shr_all + 45 * ip;
+__device__ __forceinline__ void load_sh_row(const float* __restrict__ shr_all, int64_t ip, int nsh, float shv[45]) {
+    const float* sr = shr_all + 45 * ip;
 #pragma unroll
-    for (int b = 0; b < 45; ++b) shv[b] = b < nsh ? load_as_float(sr, b) : 0.f;
+    for (int j = 0; j < 11; ++j) {
+        v4f v = {0.f, 0.f, 0.f, 0.f};
+        if (4 * j < nsh) v = *(const v4f_any*)(sr + 4 * j);   // (4 j + 3 < 45: inside the row)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) shv[4 * j + q] = v[q];
+    }
+    shv[44] = nsh > 44 ? sr[44] : 0.f;
 }
-template <>
-__device__ __forceinline__ void load_sh_row<__half>(const __half* __restrict__ shr_all, int64_t ip, int nsh,
-                                                    uint2* slot, float shv[45]) {
-    // row bytes [B, B + 90), window [a, a + 96) with a = B & ~7, o = B - a in {0, 2, 4, 6}:
-    // 11 whole 8-byte words lie inside the row; of the 12th, only its first o + 2 bytes do
-    const uint64_t B = 90u * (uint64_t)ip, a = B & ~7ull;
-    const uint32_t o = (uint32_t)(B - a);
-    const uint2* win = (const uint2*)((const char*)shr_all + a);
+__device__ __forceinline__ void load_sh_row(const __half* __restrict__ shr_all, int64_t ip, int nsh, float shv[45]) {
+    // row bytes [B, B + 90), words from a = B & ~3; o = B - a is 0 or 2. 22 whole words lie inside the row;
+    // of the 23rd, both halves when o = 2, only the lower one when o = 0
+    const uint64_t B = 90u * (uint64_t)ip, a = B & ~3ull;
+    const bool o = (B & 2u) != 0u;
+    const uint32_t* win = (const uint32_t*)((const char*)shr_all + a);
+    uint32_t w[23];
 #pragma unroll
-    for (int q = 0; q < 11; ++q) slot[q] = win[q];
-    const uint16_t* tail = (const uint16_t*)(win + 11);
-    uint16_t* stail = (uint16_t*)(slot + 11);
+    for (int j = 0; j < 5; ++j) {
+        v4u v = {0u, 0u, 0u, 0u};
+        if (nsh > 0 && 8 * j <= nsh) v = *(const v4u_any*)(win + 4 * j);
 #pragma unroll
-    for (uint32_t q = 0; q < 4; ++q)
-        if (2u * q <= o) stail[q] = tail[q];
-    const __half* h = (const __half*)((const char*)slot + o);
+        for (int q = 0; q < 4; ++q) w[4 * j + q] = v[q];
+    }
+    w[20] = w[21] = w[22] = 0u;
+    if (nsh > 39) {
+        w[20] = win[20];
+        w[21] = win[21];
+        w[22] = o ? win[22] : (uint32_t)*(const uint16_t*)(win + 22);
+    }
 #pragma unroll
-    for (int b = 0; b < 45; ++b) shv[b] = b < nsh ? __half2float(h[b]) : 0.f;
+    for (int j = 0; j < 23; ++j) {
+        const uint32_t nx = j < 22 ? w[j + 1] : 0u;
+        const uint32_t r = o ? __builtin_amdgcn_alignbit(nx, w[j], 16u) : w[j];
+        const __half2 h = __builtin_bit_cast(__half2, r);
+        shv[2 * j] = __low2float(h);
+        if (2 * j + 1 < 45) shv[2 * j + 1] = __high2float(h);
+    }
 }
 
 // Pose gradient (kernels_backward.cuh:256-269): with kPose, each thread also
 // sums dL/dmean_cam[k] * (mean, 1) over its primitives, and the workgroup's
 // sum of those 12 numbers goes to pose_partial[12 * chunk] (every workgroup
 // writes its slot, zero when it has no live primitive), in a fixed order.
-template <typename ShT, bool kPose, bool kHalf>
-__global__ void __launch_bounds__(256) preprocess_backward_chunk_kernel(
+// Latency bound (dependent loads: list, records, parameter rows); four waves
+// per SIMD (at most 128 VGPRs) hide more of it than the three the compiler
+// chose: half sums at 1M primitives 58 -> 52 us.
+template <typename ShT, bool kPose, bool kHalf, int kClassRounds>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) preprocess_backward_chunk_kernel(
     int64_t n, const uint32_t* __restrict__ n_touched, const uint32_t* __restrict__ first_slot,
     uint8_t* __restrict__ row_mask, uint4* __restrict__ live, uint4* __restrict__ heavy,
     const float* __restrict__ means, const float* __restrict__ scales, const float* __restrict__ rots,
@@ -737,12 +770,12 @@ __global__ void __launch_bounds__(256) preprocess_backward_chunk_kernel(
     uint32_t* __restrict__ rec_count, uint32_t* __restrict__ rec_mask, const uint32_t* __restrict__ rec_bits,
     uint32_t slot_limit, const float4* __restrict__ records, float* grad2d, GradView out,
     float4* __restrict__ densif, int mode, float* __restrict__ pose_partial, float* keep2d) {
+    constexpr int kClassChunk = 256 * kClassRounds;
     __shared__ uint32_t s_rw[4 * kClassRounds];
-    __shared__ uint2 s_win[256 * kShWin];
     const uint32_t t = threadIdx.x;
     // phase 1: the chunk's lists; phase 2: its heavy primitives' sums into grad2d
     uint32_t nl, nh;
-    classify_chunk<kHalf>(n, rec_count, rec_mask, first_slot, n_touched, densif, mode, row_mask, out, live, heavy,
+    classify_chunk<kHalf, kClassRounds>(n, rec_count, rec_mask, first_slot, n_touched, densif, mode, row_mask, out, live, heavy,
                           slot_limit, s_rw, nl, nh);
     __syncthreads();   // the lists (global, this chunk's slices) seen by the whole workgroup
     if (nh) {
@@ -777,7 +810,6 @@ __global__ void __launch_bounds__(256) preprocess_backward_chunk_kernel(
             float v[12];
 #pragma unroll
             for (int q = 0; q < 12; ++q) v[q] = 0.f;
-            // (the thread's SH staging slot holds its slot list until the SH row is read)
             add_marked_light(rec_bits, records, e.z, e.w, nr, e.y >> 5, v);
             gA = make_float4(v[0], v[1], v[2], v[3]);
             gB = make_float4(v[4], v[5], v[6], v[7]);
@@ -804,7 +836,7 @@ __global__ void __launch_bounds__(256) preprocess_backward_chunk_kernel(
         for (int c = 0; c < 4; ++c) pq[c] = rots[4 * ip + c];
         // half mode: the records carry (1 - opacity) already
         const float opacity = kHalf ? 0.0f : conic_opacity[ip].w;
-        load_sh_row<ShT>(shr_all, ip, nsh, s_win + kShWin * t, shv);
+        load_sh_row(shr_all, ip, nsh, shv);
         PrimGrad pg;
         float gc[3], k[15];
         for (int b = 0; b < 15; ++b) k[b] = 0.f;
@@ -847,21 +879,20 @@ __global__ void __launch_bounds__(256) preprocess_backward_chunk_kernel(
             for (int c = 0; c < 3; ++c) v[3 * b + c] = b < nb ? k[b] * gc[c] : 0.f;
         float* gr = out.sh_rest + 45 * ip;
         if (store) {
-            // row bytes [R, R + 180): s = 1 when R is 4 mod 8; 8-byte pairs at R + 4 s + 8 j
-            // hold elements (s + 2 j, s + 2 j + 1); the one element left over is 0 or 44
-            const uint32_t s1 = (uint32_t)(ip & 1);   // 180 ip = 4 ip (mod 8)
-            float2* pairs = (float2*)(gr + s1);
 #pragma unroll
-            for (int j = 0; j < 22; ++j)
-                pairs[j] = s1 ? make_float2(v[2 * j + 1], v[2 * j + 2]) : make_float2(v[2 * j], v[2 * j + 1]);
-            if (s1)
-                gr[0] = v[0];
-            else
-                gr[44] = v[44];
-        } else {
+            for (int j = 0; j < 11; ++j)
+                *(v4f_any*)(gr + 4 * j) = v4f{v[4 * j], v[4 * j + 1], v[4 * j + 2], v[4 * j + 3]};
+            gr[44] = v[44];
+        } else {   // the active bases' 9, 24 or 45 values
 #pragma unroll
-            for (int j = 0; j < 45; ++j)   // constant indices keep v in registers
-                if (j < 3 * nb) gr[j] += v[j];
+            for (int j = 0; j < 11; ++j)
+                if (4 * j + 3 < 3 * nb) {
+                    const v4f old = *(const v4f_any*)(gr + 4 * j);
+                    *(v4f_any*)(gr + 4 * j) = v4f{old[0] + v[4 * j], old[1] + v[4 * j + 1], old[2] + v[4 * j + 2],
+                                                  old[3] + v[4 * j + 3]};
+                }
+            if (nb == 3) gr[8] += v[8];
+            if (nb == 15) gr[44] += v[44];
         }
     }
     if constexpr (kPose) {
@@ -916,21 +947,25 @@ static void launch_chunks(const GaussianView& g, int bases, const CamParams& cam
                           const uint32_t* first_slot, uint8_t* row_mask, uint4* live, uint4* heavy,
                           const float4* conic_opacity, uint32_t* rec_count, uint32_t* rec_mask,
                           const uint32_t* rec_bits, uint32_t slot_limit, const float4* records, float* grad2d,
-                          const GradView& out,
-                          float* densif, int mode, float* pose_partial, bool keep2d, bool half_sums, unsigned chunks,
-                          hipStream_t s) {
+                          const GradView& out, float* densif, int mode, float* pose_partial, bool keep2d,
+                          bool half_sums, unsigned chunks, hipStream_t s) {
+    auto launch = [&](auto kernel) {
+        kernel<<<chunks, 256, 0, s>>>(g.n, n_touched, first_slot, row_mask, live, heavy, g.means, g.scales,
+                                      g.rotations, (const ShT*)g.sh_rest, bases, cam, conic_opacity, rec_count,
+                                      rec_mask, rec_bits, slot_limit, records, grad2d, out, (float4*)densif, mode,
+                                      pose_partial, keep2d ? grad2d : nullptr);
+    };
+    auto of_rounds = [&](auto half) {
+        constexpr bool kHalf = decltype(half)::value;
+        if (pb_rounds(g.n) == 1)
+            launch(preprocess_backward_chunk_kernel<ShT, kPose, kHalf, 1>);
+        else
+            launch(preprocess_backward_chunk_kernel<ShT, kPose, kHalf, kManyRounds>);
+    };
     if (half_sums)
-        preprocess_backward_chunk_kernel<ShT, kPose, true><<<chunks, 256, 0, s>>>(
-            g.n, n_touched, first_slot, row_mask, live, heavy, g.means, g.scales, g.rotations,
-            (const ShT*)g.sh_rest, bases, cam, conic_opacity, rec_count, rec_mask, rec_bits, slot_limit, records, grad2d,
-            out,
-            (float4*)densif, mode, pose_partial, keep2d ? grad2d : nullptr);
+        of_rounds(std::true_type{});
     else
-        preprocess_backward_chunk_kernel<ShT, kPose, false><<<chunks, 256, 0, s>>>(
-            g.n, n_touched, first_slot, row_mask, live, heavy, g.means, g.scales, g.rotations,
-            (const ShT*)g.sh_rest, bases, cam, conic_opacity, rec_count, rec_mask, rec_bits, slot_limit, records, grad2d,
-            out,
-            (float4*)densif, mode, pose_partial, keep2d ? grad2d : nullptr);
+        of_rounds(std::false_type{});
 }
 
 void launch_preprocess_backward(const GaussianView& g, const CamParams& cam, const uint32_t* n_touched,
