@@ -127,43 +127,76 @@ __device__ __forceinline__ void sh_to_color(const ShT* __restrict__ sh0, const S
 }
 
 // SH-rest coefficients of a workgroup's 256 primitives are one contiguous
-// run, staged in LDS with 16-byte lane-contiguous loads. sh_stage_load issues
-// the loads first and holds them in registers through the projection and the
-// tile tests; sh_stage_store writes them to LDS and synchronises the
-// workgroup just before the colour (every thread must reach it).
+// run, passed through LDS with 16-byte lane-contiguous loads in kParts parts of
+// whole rows. sh_stage_load issues the first part's loads, held in
+// registers through the projection and the tile tests; sh_stage_colors writes
+// a part to LDS, issues the next part's loads, and lets the part's own threads
+// form their colours (every thread must reach the call).
+//
+// What a workgroup holds bounds how many run on a CU, and its memory requests
+// are in flight only at its start. With fp32 rows in one part (46 KB of LDS,
+// 105 registers) three did, and the kernel moved 3.1 TB/s; in two parts (23 KB,
+// 85 registers) five do: 96 -> 82 us for 1,000,003 primitives of degree 3.
+// Four parts: 85 us (more barriers). fp16 rows stay in one part (60 us; two
+// 61, four 65): the same 23 KB.
 template <typename ShT>
 struct ShStage {
-    static constexpr int kVec = (256 * 45 * (int)sizeof(ShT) + 16 * 256 - 1) / (16 * 256);   // uint4 per thread
+    static constexpr int kParts = sizeof(ShT) == 4 ? 2 : 1;
+    static constexpr int kRows = 256 / kParts;   // rows per part
+    static constexpr int kPartVec = kRows * 45 * (int)sizeof(ShT) / 16;   // uint4 per part
+    static constexpr int kVec = (kPartVec + 255) / 256;                     // uint4 per thread and part
+    static_assert(kPartVec * 16 == kRows * 45 * (int)sizeof(ShT), "a part is whole 16-byte pieces");
     uint4 v[kVec];
-    int64_t blk0;
-    int count, nvec;
+    const ShT* run;   // the workgroup's first row
+    int count;        // its elements (0 for degree 0)
+    // whole 16-byte pieces of part p held by the run
+    __device__ __forceinline__ int pieces(int p) const {
+        return min(((count * (int)sizeof(ShT)) >> 4) - p * kPartVec, kPartVec);
+    }
+    __device__ __forceinline__ void load(int p) {
+        const uint4* s4 = (const uint4*)run + p * kPartVec;
+        const int nv = pieces(p);
+#pragma unroll
+        for (int q = 0; q < kVec; ++q) {
+            const int i = (int)threadIdx.x + 256 * q;
+            v[q] = i < nv ? s4[i] : make_uint4(0u, 0u, 0u, 0u);
+        }
+    }
 };
 
 template <typename ShT>
 __device__ __forceinline__ void sh_stage_load(ShStage<ShT>& st, const ShT* __restrict__ shr, int64_t n, int bases) {
-    st.blk0 = (int64_t)blockIdx.x * 256;
-    st.count = bases > 1 ? (int)min((int64_t)256, n - st.blk0) * 45 : 0;
-    st.nvec = (st.count * (int)sizeof(ShT)) >> 4;
-    const uint4* s4 = (const uint4*)(shr + st.blk0 * 45);
-#pragma unroll
-    for (int q = 0; q < ShStage<ShT>::kVec; ++q) {
-        const int v = (int)threadIdx.x + 256 * q;
-        st.v[q] = v < st.nvec ? s4[v] : make_uint4(0u, 0u, 0u, 0u);
-    }
+    const int64_t blk0 = (int64_t)blockIdx.x * 256;
+    st.count = bases > 1 ? (int)min((int64_t)256, n - blk0) * 45 : 0;
+    st.run = shr + blk0 * 45;
+    st.load(0);
 }
 
-template <typename ShT>
-__device__ __forceinline__ void sh_stage_store(const ShStage<ShT>& st, ShT* s_sh, const ShT* __restrict__ shr) {
-    uint4* d4 = (uint4*)s_sh;
-#pragma unroll
-    for (int q = 0; q < ShStage<ShT>::kVec; ++q) {
-        const int v = (int)threadIdx.x + 256 * q;
-        if (v < st.nvec) d4[v] = st.v[q];
+// Calls color(row) for this thread's SH-rest row.
+template <typename ShT, class Color>
+__device__ __forceinline__ void sh_stage_colors(ShStage<ShT>& st, ShT* s_sh, Color color) {
+    if (st.count == 0) {   // degree 0: no row is read
+        color(s_sh);
+        return;
     }
-    // the elements after the last whole 16 bytes
-    for (int e = (st.nvec << 4) / (int)sizeof(ShT) + (int)threadIdx.x; e < st.count; e += 256)
-        s_sh[e] = shr[st.blk0 * 45 + e];
-    __syncthreads();
+    constexpr int kRows = ShStage<ShT>::kRows, kParts = ShStage<ShT>::kParts;
+    uint4* d4 = (uint4*)s_sh;
+    const int t = (int)threadIdx.x;
+#pragma unroll
+    for (int p = 0; p < kParts; ++p) {
+        const int nv = st.pieces(p);
+        if (p > 0) __syncthreads();   // the part before it has been read
+#pragma unroll
+        for (int q = 0; q < ShStage<ShT>::kVec; ++q)
+            if (t + 256 * q < nv) d4[t + 256 * q] = st.v[q];
+        // the run's elements after its last whole 16 bytes
+        constexpr int kPartElems = kRows * 45;
+        const int e = ((st.count * (int)sizeof(ShT)) >> 4) * 16 / (int)sizeof(ShT) + t;
+        if (e < st.count && e >= p * kPartElems && e < (p + 1) * kPartElems) s_sh[e - p * kPartElems] = st.run[e];
+        if (p + 1 < kParts) st.load(p + 1);
+        __syncthreads();
+        if (t / kRows == p) color(s_sh + 45 * (t - p * kRows));
+    }
 }
 
 template <typename ShT>
@@ -173,7 +206,7 @@ __global__ void __launch_bounds__(256) preprocess_kernel(
     CamParams cam, uint32_t* __restrict__ n_touched, uint4* __restrict__ erec,
     float2* __restrict__ mean2d, float4* __restrict__ conic_opacity, float4* __restrict__ color_pt, uint32_t* __restrict__ depth_key,
     float4* __restrict__ densif, BinCtl* __restrict__ ctl) {
-    __shared__ __align__(16) ShT s_sh[256 * 45];
+    __shared__ __align__(16) ShT s_sh[ShStage<ShT>::kRows * 45];
     __shared__ uint32_t s_rect[4][kRectSlice];
     if (ctl != nullptr && blockIdx.x == 0) bin_ctl_reset_block(ctl);   // (read first by the compaction)
     ShStage<ShT> shs;
@@ -290,20 +323,20 @@ __global__ void __launch_bounds__(256) preprocess_kernel(
                         });
     }
 
-    sh_stage_store(shs, s_sh, shr);
-    if (i >= n) return;
-    if (!active || cnt == 0) {
-        n_touched[i] = 0;
-        return;
+    const bool visible = active && cnt != 0u;   // (active: i < n)
+    if (i < n) n_touched[i] = visible ? cnt : 0u;
+    if (visible) {
+        erec[i] = make_uint4(xmin | (xmax << 16), ymin | (ymax << 16), bits, 0u);
+        mean2d[i] = make_float2(m2x, m2y);
+        conic_opacity[i] = make_float4(ca, cb, cc, opacity);
+        depth_key[i] = f2u(depth);
     }
-    n_touched[i] = cnt;
-    erec[i] = make_uint4(xmin | (xmax << 16), ymin | (ymax << 16), bits, 0u);
-    mean2d[i] = make_float2(m2x, m2y);
-    conic_opacity[i] = make_float4(ca, cb, cc, opacity);
-    float col[3];
-    sh_to_color(sh0, s_sh + 45 * threadIdx.x, i, mx, my, mz, cam, bases, col);
-    color_pt[i] = make_float4(col[0], col[1], col[2], pthr);
-    depth_key[i] = f2u(depth);
+    sh_stage_colors(shs, s_sh, [&](const ShT* row) {
+        if (!visible) return;
+        float col[3];
+        sh_to_color(sh0, row, i, mx, my, mz, cam, bases, col);
+        color_pt[i] = make_float4(col[0], col[1], col[2], pthr);
+    });
 }
 
 // preprocess_cu of the fp16-image rasterizer (FGS16), tinygs/src/rasterizer/
@@ -323,7 +356,7 @@ __global__ void __launch_bounds__(256) preprocess16_kernel(
     CamParams cam, uint32_t* __restrict__ n_touched, uint4* __restrict__ erec,
     float2* __restrict__ mean2d, float4* __restrict__ conic_opacity, uint4* __restrict__ info,
     uint32_t* __restrict__ depth_key, float4* __restrict__ densif, BinCtl* __restrict__ ctl) {
-    __shared__ __align__(16) ShT s_sh[256 * 45];
+    __shared__ __align__(16) ShT s_sh[ShStage<ShT>::kRows * 45];
     __shared__ uint32_t s_rect[4][kRectSlice];
     if (ctl != nullptr && blockIdx.x == 0) bin_ctl_reset_block(ctl);   // (read first by the compaction)
     ShStage<ShT> shs;
@@ -445,24 +478,24 @@ __global__ void __launch_bounds__(256) preprocess16_kernel(
                         });
     }
 
-    sh_stage_store(shs, s_sh, shr);
-    if (i >= n) return;
-    if (!active || cnt == 0) {
-        n_touched[i] = 0;
-        return;
-    }
-    n_touched[i] = cnt;
-    erec[i] = make_uint4(xmin | (xmax << 16), ymin | (ymax << 16), bits, 0u);
+    const bool visible = active && cnt != 0u;   // (active: i < n)
+    if (i < n) n_touched[i] = visible ? cnt : 0u;
     const uint32_t c01 = (uint32_t)hbits(hca) | ((uint32_t)hbits(hcb) << 16);
     const uint32_t c2o = (uint32_t)hbits(hcc) | ((uint32_t)hbits(opacity) << 16);
-    mean2d[i] = make_float2(m2x, m2y);
-    conic_opacity[i] = make_float4((float)hca, (float)hcb, (float)hcc, (float)opacity);
-    float col[3];
-    sh_to_color(sh0, s_sh + 45 * threadIdx.x, i, mx, my, mz, cam, bases, col);
-    uint32_t rgb = 0;
-    for (int c = 0; c < 3; ++c) rgb |= (uint32_t)(uint8_t)(saturate(col[c]) * 255.0f) << (8 * c);
-    info[i] = make_uint4(c01, c2o, rgb, f2u(pthr));
-    depth_key[i] = f2u(depth);
+    if (visible) {
+        erec[i] = make_uint4(xmin | (xmax << 16), ymin | (ymax << 16), bits, 0u);
+        mean2d[i] = make_float2(m2x, m2y);
+        conic_opacity[i] = make_float4((float)hca, (float)hcb, (float)hcc, (float)opacity);
+        depth_key[i] = f2u(depth);
+    }
+    sh_stage_colors(shs, s_sh, [&](const ShT* row) {
+        if (!visible) return;
+        float col[3];
+        sh_to_color(sh0, row, i, mx, my, mz, cam, bases, col);
+        uint32_t rgb = 0;
+        for (int c = 0; c < 3; ++c) rgb |= (uint32_t)(uint8_t)(saturate(col[c]) * 255.0f) << (8 * c);
+        info[i] = make_uint4(c01, c2o, rgb, f2u(pthr));
+    });
 }
 
 void launch_preprocess16(const GaussianView& g, const CamParams& cam, uint32_t* n_touched, uint4* erec,
