@@ -670,39 +670,15 @@ int64_t record_bit_words(int64_t max_inst) {
 
 // ---------------------------------------------------------------- instance emission
 
-// kernels_forward.cuh:49-84 (same expression as in preprocess.hip)
-__device__ __forceinline__ bool will_contribute_e(float mx, float my, float ca, float cb, float cc, uint32_t tile_x,
-                                                  uint32_t tile_y, float power_threshold) {
-    const float rminx = (float)(tile_x * 16u), rminy = (float)(tile_y * 16u);
-    const float rmaxx = (float)((tile_x + 1u) * 16u - 1u), rmaxy = (float)((tile_y + 1u) * 16u - 1u);
-    const float x_min_diff = rminx - mx;
-    const float x_left = x_min_diff > 0.0f ? 1.0f : 0.0f;
-    const float not_in_x = x_left + (mx > rmaxx ? 1.0f : 0.0f);
-    const float y_min_diff = rminy - my;
-    const float y_above = y_min_diff > 0.0f ? 1.0f : 0.0f;
-    const float not_in_y = y_above + (my > rmaxy ? 1.0f : 0.0f);
-    if (not_in_y + not_in_x == 0.0f) return true;
-    const float ccx = rmaxx + x_left * (rminx - rmaxx);
-    const float ccy = rmaxy + y_above * (rminy - rmaxy);
-    const float diffx = mx - ccx, diffy = my - ccy;
-    const float dx = __builtin_copysignf(15.0f, x_min_diff);
-    const float dy = __builtin_copysignf(15.0f, y_min_diff);
-    const float tx = not_in_y * saturate((dx * ca * diffx + dx * cb * diffy) / (dx * ca * dx));
-    const float ty = not_in_x * saturate((dy * cb * diffx + dy * cc * diffy) / (dy * cc * dy));
-    const float px = ccx + tx * dx, py = ccy + ty * dy;
-    const float ddx = mx - px, ddy = my - py;
-    const float max_power = 0.5f * (ca * ddx * ddx + cc * ddy * ddy) + cb * ddx * ddy;
-    return max_power <= power_threshold;
-}
-
 // Thread per depth-sorted primitive: its 16-byte emission record (bounds and
 // the preprocess's outcomes for rect tiles 0..31) is gathered once, its mean,
-// conic and threshold only for primitives with more than 32 rect tiles (from
-// the blend's own per-primitive arrays); its instances fill the slots [offs[k], offs[k + 1]),
+// conic and threshold only for big rects (from the blend's own per-primitive
+// arrays); its instances fill the slots [offs[k], offs[k + 1]),
 // so the instance array comes out in depth order. (The gathers are random:
 // depth order is not index order, and each costs a whole memory line.) The
 // rect tiles of a wave's 64 primitives are walked as one task list, 64 per
-// step, whatever the rect sizes.
+// step, whatever the rect sizes, except big rects, walked one by one
+// (rect_tasks.h): 463 -> 324 us for 375k primitives of about 200 tiles each.
 // The workgroup's 256 primitives own one contiguous slot range; when it fits
 // in LDS the instances are staged there and written out by consecutive
 // threads (contiguous stores), otherwise written directly. 2048 slots (256
@@ -712,14 +688,15 @@ constexpr uint32_t kEmitStage = 2048;
 
 // The tile test of the record's rasterizer: fp32 (conic floats in w0..w2) or
 // FGS16 (half conic a | b << 16 in w0, c | opacity << 16 in w1).
+// ia, ic: the fp32 test's reciprocals.
 template <bool kHalf>
-__device__ __forceinline__ bool emit_test(float mx, float my, uint32_t w0, uint32_t w1, uint32_t w2, uint32_t tx,
-                                          uint32_t ty, float pt) {
+__device__ __forceinline__ bool emit_test(float mx, float my, uint32_t w0, uint32_t w1, uint32_t w2, float ia,
+                                          float ic, uint32_t tx, uint32_t ty, float pt) {
     if constexpr (kHalf)
         return will_contribute_half(mx, my, hfrom((uint16_t)(w0 & 0xffffu)), hfrom((uint16_t)(w0 >> 16)),
                                     hfrom((uint16_t)(w1 & 0xffffu)), tx, ty, pt);
     else
-        return will_contribute_e(mx, my, u2f(w0), u2f(w1), u2f(w2), tx, ty, pt);
+        return will_contribute(mx, my, u2f(w0), u2f(w1), u2f(w2), ia, ic, tx, ty, pt);
 }
 
 template <bool kHalf>
@@ -770,7 +747,7 @@ __global__ void __launch_bounds__(256) emit_kernel(const uint32_t* __restrict__ 
     const bool active = k < n;
     const uint32_t lane = lane_id();
     uint32_t p = 0, off = 0, cap = 0, x0 = 0, x1 = 0, y0 = 0, y1 = 0, bits = 0;
-    float smx = 0.f, smy = 0.f, pt = 0.f;
+    float smx = 0.f, smy = 0.f, pt = 0.f, ia = 0.f, ic = 0.f;
     uint32_t cw0 = 0, cw1 = 0, cw2 = 0;
     if (active) {
         p = prims[k];
@@ -783,22 +760,33 @@ __global__ void __launch_bounds__(256) emit_kernel(const uint32_t* __restrict__ 
         const uint4 e = erec[p];
         x0 = e.x & 0xffffu; x1 = e.x >> 16; y0 = e.y & 0xffffu; y1 = e.y >> 16;
         bits = e.z;
-        if ((x1 - x0) * (y1 - y0) > 32u) {   // tiles past the first 32 need the exact test
+        if ((x1 - x0) * (y1 - y0) > kBigRect) {   // the exact test's values
             const float2 m = mean2d[p];
             const uint4 cw = conic_words[p];
             smx = m.x - 0.5f;
             smy = m.y - 0.5f;
             cw0 = cw.x; cw1 = cw.y; cw2 = cw.z;
             pt = u2f(kHalf ? cw.w : thr_words[p].w);
+            if constexpr (!kHalf) {
+                ia = tile_test_inverse(u2f(cw0));
+                ic = tile_test_inverse(u2f(cw2));
+            }
         }
     }
-    // The wave's rect tiles as one task list (rect_tasks.h); rect tiles
-    // 0..31 were tested by the preprocess (emission record). A hit's slot is
-    // its primitive's first slot plus the number of its hits before it: the
-    // hits in earlier windows (only the primitive carried into the window has
-    // any) and those of this window on lower lanes of its segment.
+    // fp32 images: the key's bits from 16 up carry the instance's rank among
+    // its primitive's instances (tile keys there are below 2^16)
+    auto key_of = [&](uint32_t tx, uint32_t ty, uint32_t rank) {
+        return (ty * grid_w + tx) | (kHalf ? 0u : rank << 16);
+    };
+    // The wave's rect tiles as one task list (rect_tasks.h); rects of up to
+    // kBigRect tiles were tested by the preprocess (emission record). A hit's
+    // slot is its primitive's first slot plus the number of its hits before
+    // it: the hits in earlier windows (only the primitive carried into the
+    // window has any) and those of this window on lower lanes of its segment.
     const uint32_t bw = x1 - x0;
-    const uint32_t nr = active ? bw * (y1 - y0) : 0u;
+    const uint32_t nrect = active ? bw * (y1 - y0) : 0u;
+    const bool big = nrect > kBigRect;
+    const uint32_t nr = big ? 0u : nrect;
     const uint32_t incl = wave_inclusive_scan_u32(nr);
     const uint32_t total = readlane_u32(incl, 63);
     const uint32_t ex = incl - nr, org = x0 | (y0 << 16), end = off + cap;
@@ -819,25 +807,35 @@ __global__ void __launch_bounds__(256) emit_kernel(const uint32_t* __restrict__ 
             rect_tile_of(q, wj, col, row);
             tx = (orgj & 0xffffu) + col;
             ty = (orgj >> 16) + row;
-            hit = q < 32u && ((bitsj >> q) & 1u) != 0u;
-        }
-        if (ballot(tt < total && q >= 32u)) {   // the exact test, with the owner's record
-            const float s_mx = u2f(lane_gather(j, f2u(smx))), s_my = u2f(lane_gather(j, f2u(smy)));
-            const uint32_t s_a = lane_gather(j, cw0), s_b = lane_gather(j, cw1), s_c = lane_gather(j, cw2);
-            const float s_t = u2f(lane_gather(j, f2u(pt)));
-            if (tt < total && q >= 32u) hit = emit_test<kHalf>(s_mx, s_my, s_a, s_b, s_c, tx, ty, s_t);
+            hit = ((bitsj >> q) & 1u) != 0u;   // q < kBigRect
         }
         const uint64_t hm = ballot(hit);
         const uint32_t seg = exj > base ? exj - base : 0u;   // the owner's first lane in this window
         const uint64_t below = hm & ((1ull << lane) - 1ull) & ~((1ull << seg) - 1ull);
         const uint32_t pos = offj + (j + 1u == prev ? carry_hits : 0u) + (uint32_t)__builtin_popcountll(below);
-        // fp32 images: the key's bits from 16 up carry the instance's rank
-        // among its primitive's instances (tile keys there are below 2^16)
-        if (hit && pos < endj) put(pos, (ty * grid_w + tx) | (kHalf ? 0u : (pos - offj) << 16), pj);
+        if (hit && pos < endj) put(pos, key_of(tx, ty, pos - offj), pj);
         // hits so far of the primitive carried into the next window (lane 63's owner)
         const uint32_t seg63 = readlane_u32(seg, 63);
         const uint32_t h63 = (uint32_t)__builtin_popcountll(hm & ~((1ull << seg63) - 1ull));
         carry_hits = (carry == prev ? carry_hits : 0u) + h63;
+    }
+    // big rects one by one: a hit's slot follows the rect's earlier hits
+    for (uint64_t todo = ballot(big); todo != 0ull; todo &= todo - 1ull) {
+        const uint32_t j = (uint32_t)__builtin_ctzll(todo);
+        const float jmx = readlane_f32(smx, j), jmy = readlane_f32(smy, j), jpt = readlane_f32(pt, j);
+        const uint32_t jw0 = readlane_u32(cw0, j), jw1 = readlane_u32(cw1, j), jw2 = readlane_u32(cw2, j);
+        const float jia = readlane_f32(ia, j), jic = readlane_f32(ic, j);
+        const uint32_t jp = readlane_u32(p, j), joff = readlane_u32(off, j), jend = readlane_u32(end, j);
+        uint32_t done = 0;
+        walk_big_rect(readlane_u32(nrect, j), readlane_u32(org, j), readlane_u32(bw, j),
+                      [&](uint32_t, bool valid, uint32_t tx, uint32_t ty) {
+                          const bool hit =
+                              valid && emit_test<kHalf>(jmx, jmy, jw0, jw1, jw2, jia, jic, tx, ty, jpt);
+                          const uint64_t hm = ballot(hit);
+                          const uint32_t rank = done + mask_rank(hm);
+                          if (hit && joff + rank < jend) put(joff + rank, key_of(tx, ty, rank), jp);
+                          done += (uint32_t)__builtin_popcountll(hm);
+                      });
     }
     if (staged) {
         __syncthreads();

@@ -21,36 +21,17 @@
 
 namespace tgs {
 
-// kernels_forward.cuh:49-84, on the mean shifted by -0.5 (:94).
-__device__ __forceinline__ bool will_contribute(float mx, float my, float ca, float cb, float cc, uint32_t tile_x,
-                                                uint32_t tile_y, float power_threshold) {
-    const float rminx = (float)(tile_x * 16u), rminy = (float)(tile_y * 16u);
-    const float rmaxx = (float)((tile_x + 1u) * 16u - 1u), rmaxy = (float)((tile_y + 1u) * 16u - 1u);
-    const float x_min_diff = rminx - mx;
-    const float x_left = x_min_diff > 0.0f ? 1.0f : 0.0f;
-    const float not_in_x = x_left + (mx > rmaxx ? 1.0f : 0.0f);
-    const float y_min_diff = rminy - my;
-    const float y_above = y_min_diff > 0.0f ? 1.0f : 0.0f;
-    const float not_in_y = y_above + (my > rmaxy ? 1.0f : 0.0f);
-    if (not_in_y + not_in_x == 0.0f) return true;
-    const float ccx = rmaxx + x_left * (rminx - rmaxx);
-    const float ccy = rmaxy + y_above * (rminy - rmaxy);
-    const float diffx = mx - ccx, diffy = my - ccy;
-    const float dx = __builtin_copysignf(15.0f, x_min_diff);
-    const float dy = __builtin_copysignf(15.0f, y_min_diff);
-    const float tx = not_in_y * saturate((dx * ca * diffx + dx * cb * diffy) / (dx * ca * dx));
-    const float ty = not_in_x * saturate((dy * cb * diffx + dy * cc * diffy) / (dy * cc * dy));
-    const float px = ccx + tx * dx, py = ccy + ty * dy;
-    const float ddx = mx - px, ddy = my - py;
-    const float max_power = 0.5f * (ca * ddx * ddx + cc * ddy * ddy) + cb * ddx * ddy;
-    return max_power <= power_threshold;
-}
-
-// Exact tile counts of the wave's 64 primitives, their rect tiles spread over
-// the wave's lanes (rect_tasks.h). Hits are counted, and the outcomes of rect
-// tiles 0..31 kept as a bit mask, with LDS atomics: the results do not depend
-// on the order of the tests. test(par, tile_x, tile_y) sees the owner's NP
-// parameter words. s: this wave's kRectSlice words. Called by the whole wave.
+// Exact tile counts of the wave's 64 primitives: big rects one by one, the
+// others spread over the wave's lanes as one task list (rect_tasks.h). The
+// list's hits are counted, and the outcomes of rect tiles 0..31 kept as a bit
+// mask, with LDS atomics: the results do not depend on the order of the tests.
+// test(par, tile_x, tile_y) sees the owner's NP parameter words. s: this
+// wave's kRectSlice words. Called by the whole wave.
+//
+// The windows' instructions and LDS latency bound this. With every rect in the
+// list, and a division per quotient, the kernel took 558 us for 375k
+// primitives of about 200 tiles each (now 322) and 116 us for 500k of about 20
+// (now 89).
 constexpr int kRectSlice = 3 * 64;
 
 template <int NP, class Test>
@@ -61,32 +42,48 @@ __device__ __forceinline__ void wave_rect_tests(uint32_t nrect, uint32_t xmin, u
     uint32_t* s_mark = s;
     uint32_t* s_cnt = s + 64;
     uint32_t* s_bits = s + 128;
-    const uint32_t incl = wave_inclusive_scan_u32(nrect);
+    const bool big = nrect > kBigRect;
+    const uint32_t nlist = big ? 0u : nrect;
+    const uint32_t incl = wave_inclusive_scan_u32(nlist);
     const uint32_t total = readlane_u32(incl, 63);
-    const uint32_t ex = incl - nrect, org = xmin | (ymin << 16);
+    const uint32_t ex = incl - nlist, org = xmin | (ymin << 16);
     s_cnt[lane] = 0u;
     s_bits[lane] = 0u;
     uint32_t carry = 0;
     for (uint32_t base = 0; base < total; base += kWave) {
-        const uint32_t j = wave_task_owner(s_mark, nrect, ex, base, carry);
+        const uint32_t j = wave_task_owner(s_mark, nlist, ex, base, carry);
         const uint32_t exj = lane_gather(j, ex), orgj = lane_gather(j, org), w = lane_gather(j, bw);
         uint32_t pj[NP];
 #pragma unroll
         for (int q = 0; q < NP; ++q) pj[q] = lane_gather(j, par[q]);
         const uint32_t t = base + lane;
         if (t < total) {
-            const uint32_t k = t - exj;
+            const uint32_t k = t - exj;   // < kBigRect
             uint32_t col, row;
             rect_tile_of(k, w, col, row);
             if (test(pj, (orgj & 0xffffu) + col, (orgj >> 16) + row)) {
                 atomicAdd(&s_cnt[j], 1u);
-                if (k < 32u) atomicOr(&s_bits[j], 1u << k);
+                atomicOr(&s_bits[j], 1u << k);
             }
         }
     }
     wave_lds_sync();
     cnt = s_cnt[lane];
     bits = s_bits[lane];
+    for (uint64_t todo = ballot(big); todo != 0ull; todo &= todo - 1ull) {
+        const uint32_t j = (uint32_t)__builtin_ctzll(todo);
+        uint32_t pj[NP], c = 0, b = 0;
+#pragma unroll
+        for (int q = 0; q < NP; ++q) pj[q] = readlane_u32(par[q], j);
+        walk_big_rect(readlane_u32(nrect, j), readlane_u32(org, j), readlane_u32(bw, j),
+                      [&](uint32_t first, bool valid, uint32_t tx, uint32_t ty) {
+                          const uint64_t hits = ballot(valid && test(pj, tx, ty));
+                          if (first == 0u) b = (uint32_t)hits;
+                          c += (uint32_t)__builtin_popcountll(hits);
+                      });
+        cnt = lane == j ? c : cnt;
+        bits = lane == j ? b : bits;
+    }
 }
 
 template <typename ShT>
@@ -315,11 +312,12 @@ __global__ void __launch_bounds__(256) preprocess_kernel(
     const float smx = m2x - 0.5f, smy = m2y - 0.5f;
     uint32_t cnt = 0, bits = 0;
     {
-        const uint32_t par[6] = {f2u(smx), f2u(smy), f2u(ca), f2u(cb), f2u(cc), f2u(pthr)};
+        const uint32_t par[8] = {f2u(smx), f2u(smy), f2u(ca), f2u(cb), f2u(cc), f2u(pthr),
+                                 f2u(tile_test_inverse(ca)), f2u(tile_test_inverse(cc))};
         wave_rect_tests(active ? nmax : 0u, xmin, ymin, xmax - xmin, par, s_rect[threadIdx.x >> 6], cnt, bits,
-                        [&](const uint32_t(&pj)[6], uint32_t tx_, uint32_t ty_) {
-                            return will_contribute(u2f(pj[0]), u2f(pj[1]), u2f(pj[2]), u2f(pj[3]), u2f(pj[4]), tx_,
-                                                   ty_, u2f(pj[5]));
+                        [&](const uint32_t(&pj)[8], uint32_t tx_, uint32_t ty_) {
+                            return will_contribute(u2f(pj[0]), u2f(pj[1]), u2f(pj[2]), u2f(pj[3]), u2f(pj[4]),
+                                                   u2f(pj[6]), u2f(pj[7]), tx_, ty_, u2f(pj[5]));
                         });
     }
 

@@ -9,6 +9,10 @@
 // starts inside the window marks its start position in LDS, and a prefix
 // maximum over the window, carrying the previous window's last owner, spreads
 // the marks. The owner's values then come over ds_bpermute.
+//
+// A rect of more than kBigRect tiles is walked by the whole wave instead, 64
+// tiles per step: its values are wave-uniform (scalar registers), so nothing
+// is gathered or marked, and its hits are counted by ballot.
 #pragma once
 #include "common.h"
 
@@ -60,6 +64,78 @@ __device__ __forceinline__ void rect_tile_of(uint32_t k, uint32_t w, uint32_t& c
     }
     col = (uint32_t)r;
     row = q;
+}
+
+// Rects of more tiles than this are walked one by one. The emission keeps the
+// preprocess's outcomes of the first 32 tiles, so its task list then needs no
+// tile test; a walk of one step costs less than half a window of tasks, which
+// puts the break-even at about half a step, 32 tiles, as well.
+constexpr uint32_t kBigRect = 32u;
+
+// Calls step(first, valid, tile x, tile y) for the tiles of one big rect, 64 per
+// step (tile first + lane); the arguments are wave-uniform. Columns and rows
+// advance by 64 / w and 64 % w, exact for any rect.
+template <class Step>
+__device__ __forceinline__ void walk_big_rect(uint32_t n, uint32_t org, uint32_t w, Step step) {
+    uint32_t col, row, dcol, drow;
+    rect_tile_of(lane_id(), w, col, row);
+    rect_tile_of((uint32_t)kWave, w, dcol, drow);
+    for (uint32_t first = 0; first < n; first += (uint32_t)kWave) {
+        step(first, first + lane_id() < n, (org & 0xffffu) + col, (org >> 16) + row);
+        col += dcol;
+        row += drow;
+        if (col >= w) {
+            col -= w;
+            ++row;
+        }
+    }
+}
+
+// RN(a / b) for y = RN(1 / b), or by division where y is 0: two residual
+// corrections of a y (P. Markstein, "Computation of elementary functions on
+// the IBM RISC System/6000 processor", 1990: the second starts within one unit
+// in the last place of the quotient, so it rounds correctly). y is 0 unless
+// 2^-40 <= |b| <= 2^40 (tile_test_inverse) and |a| is checked here, so no
+// residual or quotient leaves the normal range. Five operations instead of the
+// division's eleven.
+TGS_HD float quotient_by(float a, float b, float y) {
+    const float m = __builtin_fabsf(a);
+    if (!(y != 0.0f && m >= 0x1p-60f && m <= 0x1p60f)) return a / b;
+    float q = a * y;
+    q = __builtin_fmaf(__builtin_fmaf(-b, q, a), y, q);
+    return __builtin_fmaf(__builtin_fmaf(-b, q, a), y, q);
+}
+
+// The divisor of the tile test along an axis with conic diagonal c: (dx c) dx
+// for dx = +-15, the same value for both signs; and its reciprocal as
+// quotient_by takes it.
+TGS_HD float tile_test_divisor(float c) { return (15.0f * c) * 15.0f; }
+TGS_HD float tile_test_inverse(float c) {
+    const float b = tile_test_divisor(c), m = __builtin_fabsf(b);
+    return m >= 0x1p-40f && m <= 0x1p40f ? 1.0f / b : 0.0f;
+}
+
+// kernels_forward.cuh:49-84, on the mean shifted by -0.5 (:94): whether the
+// primitive may contribute to a tile. ia, ic: tile_test_inverse of ca and cc.
+__device__ __forceinline__ bool will_contribute(float mx, float my, float ca, float cb, float cc, float ia, float ic,
+                                                uint32_t tile_x, uint32_t tile_y, float power_threshold) {
+    const float rminx = (float)(tile_x * 16u), rminy = (float)(tile_y * 16u);
+    const float rmaxx = rminx + 15.0f, rmaxy = rminy + 15.0f;
+    const float x_min_diff = rminx - mx, y_min_diff = rminy - my;
+    const bool left = x_min_diff > 0.0f, above = y_min_diff > 0.0f;
+    const bool out_x = left || mx > rmaxx, out_y = above || my > rmaxy;
+    // the tile corner nearest the mean
+    const float ccx = left ? rminx : rmaxx, ccy = above ? rminy : rmaxy;
+    const float diffx = mx - ccx, diffy = my - ccy;
+    const float dx = __builtin_copysignf(15.0f, x_min_diff);
+    const float dy = __builtin_copysignf(15.0f, y_min_diff);
+    const float qx = quotient_by(dx * ca * diffx + dx * cb * diffy, tile_test_divisor(ca), ia);
+    const float qy = quotient_by(dy * cb * diffx + dy * cc * diffy, tile_test_divisor(cc), ic);
+    const float tx = out_y ? saturate(qx) : 0.0f, ty = out_x ? saturate(qy) : 0.0f;
+    const float px = ccx + tx * dx, py = ccy + ty * dy;
+    const float ddx = mx - px, ddy = my - py;
+    const float max_power = 0.5f * (ca * ddx * ddx + cc * ddy * ddy) + cb * ddx * ddy;
+    return !(out_x || out_y) || max_power <= power_threshold;
 }
 
 }  // namespace tgs

@@ -3,6 +3,7 @@
 // (checked against plain host arithmetic).
 #include "common.h"
 #include "kernels.h"
+#include "rect_tasks.h"
 
 namespace tgs {
 
@@ -250,6 +251,11 @@ __global__ void __launch_bounds__(256) clock_probe_kernel(unsigned long long* ou
 
 void launch_clock_probe(unsigned long long* out, uint32_t blocks, uint32_t iters, hipStream_t s) {
     clock_probe_kernel<<<blocks, 256, 0, s>>>(out, iters, 1.0f);
+}
+
+// Host evaluation of the tile test's quotients a / ((15 c) 15) (rect_tasks.h).
+void tile_test_quotients(const float* a, const float* c, float* out, int64_t n) {
+    for (int64_t i = 0; i < n; ++i) out[i] = quotient_by(a[i], tile_test_divisor(c[i]), tile_test_inverse(c[i]));
 }
 
 }  // namespace tgs
