@@ -663,6 +663,246 @@ int radix_sort(uint32_t* keys[2], uint32_t* vals[2], uint32_t* v2[2], const uint
         first_block_n, nullptr, offs_done, ranges, n_tiles, ranges_done, ranks, clear_bits, s);
 }
 
+// ---------------------------------------------------------------- small sorts
+
+// A forward of few primitives or instances is a chain of launches with almost
+// nothing in each: the depth sort alone is nine (compaction, then counts, scan
+// and scatter per pass), about 2 us each before any key moves. Up to
+// kSmallSort primitives, or kSmallTileSort instances, one workgroup of 16 waves
+// holds everything in LDS and runs all passes itself; keys stay in registers
+// between a pass's ranking and its scatter, so a pass is a few LDS round trips.
+// Renders through these sorts against the many-launch ones: 64 against 90 us
+// (1000 primitives, 1012 instances), 88 against 102 (6000, 10418), and at the
+// limits 92 (8192, 15290) against 102 (8193, 15294). Above, one workgroup's LDS
+// and ranking time no longer pay.
+constexpr int kSmallWaves = 16;
+constexpr int kSmallThreads = 64 * kSmallWaves;
+constexpr int kSmallKpt = 8, kSmallTileKpt = 16;   // largest keys per thread
+constexpr int64_t kSmallSort = kSmallThreads * kSmallKpt;
+constexpr int64_t kSmallTileSort = kSmallThreads * kSmallTileKpt;
+// one workgroup also initialises the tile ranges: 64 KB of them at most
+constexpr uint32_t kSmallSortTiles = 8192;
+
+struct SmallPasses {
+    int n;
+    int shift[4], bits[4];
+};
+
+// LDS positions of this thread's keys (wave w owns 64 KPT consecutive ones, as
+// rank_keys) in the order of one digit. Returns the number of valid keys.
+// s_cnt is this call's to overwrite; callers place a barrier before reusing it.
+template <int KPT, int MAXB>
+__device__ __forceinline__ uint32_t small_pass(const uint32_t (&key)[KPT], const bool (&valid)[KPT], int shift,
+                                               int bits, uint32_t (*s_cnt)[MAXB], uint32_t* s_wave,
+                                               uint32_t (&pos)[KPT]) {
+    const uint32_t t = threadIdx.x, w = t >> 6;
+    const uint32_t bins = 1u << bits, dmask = bins - 1u;
+    for (uint32_t e = t; e < (uint32_t)kSmallWaves << bits; e += kSmallThreads) s_cnt[e >> bits][e & dmask] = 0u;
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < KPT; ++r) {
+        const uint32_t d = (key[r] >> shift) & dmask;
+        const uint64_t peers = match_digit(d, bits, valid[r]);
+        const uint32_t rank = mask_rank(peers);
+        const uint32_t running = s_cnt[w][d];
+        pos[r] = running + rank;
+        if (valid[r] && rank == 0u) s_cnt[w][d] = running + (uint32_t)__builtin_popcountll(peers);
+    }
+    __syncthreads();
+    uint32_t c[kSmallWaves], sum = 0, total;
+#pragma unroll
+    for (int k = 0; k < kSmallWaves; ++k) {
+        c[k] = t < bins ? s_cnt[k][t] : 0u;
+        sum += c[k];
+    }
+    uint32_t run = block_exclusive_scan<kSmallWaves>(sum, s_wave, &total);
+    if (t < bins) {
+#pragma unroll
+        for (int k = 0; k < kSmallWaves; ++k) {
+            s_cnt[k][t] = run;
+            run += c[k];
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < KPT; ++r) pos[r] += s_cnt[w][(key[r] >> shift) & dmask];
+    return total;
+}
+
+// Visible primitives of n <= 1024 KPT in depth order (stable in the index),
+// their keys, and the instance offsets; V and I into ctl.
+template <int KPT>
+__global__ void __launch_bounds__(kSmallThreads) small_depth_sort_kernel(
+    const uint32_t* __restrict__ n_touched, const uint32_t* __restrict__ depth_key, uint32_t n, uint32_t key_base,
+    SmallPasses ps, uint32_t* __restrict__ keys_out, uint32_t* __restrict__ vals_out, uint32_t* __restrict__ offs,
+    BinCtl* __restrict__ ctl) {
+    constexpr int kMax = kSmallThreads * KPT;
+    __shared__ uint32_t s_cnt[kSmallWaves][kDepthMaxDigits];
+    __shared__ uint32_t s_key[kMax], s_nt[kMax];   // s_nt by primitive
+    __shared__ uint16_t s_val[kMax];
+    __shared__ uint32_t s_wave[kSmallWaves];
+    static_assert(kMax <= kSmallWaves * kDepthMaxDigits && kMax <= 65536, "offsets fit in s_cnt, indices in 16 bits");
+    const uint32_t t = threadIdx.x, lane = t & 63u;
+    const uint32_t base = (t >> 6) * (64u * KPT) + lane;
+    uint32_t key[KPT], val[KPT], pos[KPT], count = 0;
+    bool valid[KPT];
+#pragma unroll
+    for (int r = 0; r < KPT; ++r) {
+        const uint32_t i = base + 64u * r;
+        const uint32_t nt = i < n ? n_touched[i] : 0u;
+        key[r] = i < n ? depth_key[i] - key_base : 0u;
+        val[r] = i;
+        valid[r] = nt > 0u;
+        s_nt[i] = nt;
+    }
+    for (int p = 0; p < ps.n; ++p) {
+        if (p > 0) {
+#pragma unroll
+            for (int r = 0; r < KPT; ++r) {
+                const uint32_t i = base + 64u * r;
+                valid[r] = i < count;
+                key[r] = valid[r] ? s_key[i] : 0u;
+                val[r] = valid[r] ? s_val[i] : 0u;
+            }
+        }
+        count = small_pass<KPT, kDepthMaxDigits>(key, valid, ps.shift[p], ps.bits[p], s_cnt, s_wave, pos);
+#pragma unroll
+        for (int r = 0; r < KPT; ++r)
+            if (valid[r]) {
+                s_key[pos[r]] = key[r];
+                s_val[pos[r]] = (uint16_t)val[r];
+            }
+        __syncthreads();
+    }
+    // offsets: thread t sums the positions KPT t .. KPT t + KPT - 1
+    uint32_t* s_off = &s_cnt[0][0];
+    uint32_t nt[KPT], sum = 0, total;
+#pragma unroll
+    for (int r = 0; r < KPT; ++r) {
+        const uint32_t i = t * KPT + r;
+        nt[r] = i < count ? s_nt[s_val[i]] : 0u;
+        sum += nt[r];
+    }
+    uint32_t run = block_exclusive_scan<kSmallWaves>(sum, s_wave, &total);
+#pragma unroll
+    for (int r = 0; r < KPT; ++r) {
+        s_off[t * KPT + r] = run;
+        run += nt[r];
+    }
+    __syncthreads();
+    for (uint32_t i = t; i < count; i += kSmallThreads) {
+        keys_out[i] = s_key[i];
+        vals_out[i] = s_val[i];
+        offs[i] = s_off[i];
+    }
+    if (t == 0) {
+        offs[count] = total;
+        ctl->V = count;
+        ctl->I = total;
+    }
+}
+
+// The instances of a forward of at most 1024 KPT in tile order, the tiles'
+// ranges, the ranks (fp32 images) and the cleared record bits, as the last
+// downsweep and the first upsweep of the tile sort leave them.
+template <int KPT>
+__global__ void __launch_bounds__(kSmallThreads) small_tile_sort_kernel(
+    const uint32_t* __restrict__ keys, const uint32_t* __restrict__ vals, const uint32_t* d_n, int64_t max_n,
+    SmallPasses ps, uint32_t* __restrict__ vals_out, uint2* __restrict__ ranges, uint32_t n_tiles,
+    uint16_t* __restrict__ ranks, uint32_t* __restrict__ clear_bits, uint32_t clear_words) {
+    constexpr int kMax = kSmallThreads * KPT;
+    __shared__ uint32_t s_cnt[kSmallWaves][kTileMaxDigits];
+    __shared__ uint32_t s_key[kMax], s_val[kMax];
+    __shared__ uint32_t s_wave[kSmallWaves];
+    const uint32_t t = threadIdx.x, lane = t & 63u;
+    const uint32_t base = (t >> 6) * (64u * KPT) + lane;
+    const uint32_t n = (uint32_t)resolve_n(d_n, max_n);   // <= kMax (the launch's max_n)
+    for (uint32_t j = t; j < n_tiles; j += kSmallThreads) ranges[j] = make_uint2(0xffffffffu, 0u);
+    if (clear_bits)
+        for (uint32_t j = t; j < clear_words; j += kSmallThreads) clear_bits[j] = 0u;
+    uint32_t key[KPT], val[KPT], pos[KPT], tbits = 0;
+    bool valid[KPT];
+#pragma unroll
+    for (int r = 0; r < KPT; ++r) {
+        const uint32_t i = base + 64u * r;
+        valid[r] = i < n;
+        key[r] = valid[r] ? keys[i] : 0u;
+        val[r] = valid[r] ? vals[i] : 0u;
+    }
+    for (int p = 0; p < ps.n; ++p) {
+        if (p > 0) {
+#pragma unroll
+            for (int r = 0; r < KPT; ++r) {
+                const uint32_t i = base + 64u * r;
+                key[r] = valid[r] ? s_key[i] : 0u;
+                val[r] = valid[r] ? s_val[i] : 0u;
+            }
+        }
+        small_pass<KPT, kTileMaxDigits>(key, valid, ps.shift[p], ps.bits[p], s_cnt, s_wave, pos);
+#pragma unroll
+        for (int r = 0; r < KPT; ++r)
+            if (valid[r]) {
+                s_key[pos[r]] = key[r];
+                s_val[pos[r]] = val[r];
+            }
+        tbits += (uint32_t)ps.bits[p];
+        __syncthreads();   // (also orders the ranges' initial values before the ones below)
+    }
+    // the key's sorted bits are the tile, its bits from 16 up the rank
+    const uint32_t tmask = (1u << tbits) - 1u;
+    for (uint32_t i = t; i < n; i += kSmallThreads) {
+        const uint32_t k = s_key[i], tk = k & tmask;
+        vals_out[i] = s_val[i];
+        if (ranks) ranks[i] = (uint16_t)(k >> 16);
+        if (tk < n_tiles) {
+            if (i == 0u || (s_key[i - 1u] & tmask) != tk) ranges[tk].x = i;
+            if (i + 1u == n || (s_key[i + 1u] & tmask) != tk) ranges[tk].y = i + 1u;
+        }
+    }
+}
+
+static SmallPasses small_passes(int n_passes, const int* shifts, const int* bits) {
+    SmallPasses ps{};
+    ps.n = n_passes;
+    for (int p = 0; p < n_passes; ++p) {
+        ps.shift[p] = shifts[p];
+        ps.bits[p] = bits[p];
+    }
+    return ps;
+}
+
+bool small_depth_sort(const uint32_t* n_touched, const uint32_t* depth_key, int64_t n, uint32_t key_base,
+                      int n_passes, const int* shifts, const int* bits, uint32_t* keys_out, uint32_t* vals_out,
+                      uint32_t* offs, BinCtl* ctl, hipStream_t s) {
+    if (n <= 0 || n > kSmallSort) return false;
+    const SmallPasses ps = small_passes(n_passes, shifts, bits);
+    auto go = [&](auto kernel) {
+        kernel<<<1, kSmallThreads, 0, s>>>(n_touched, depth_key, (uint32_t)n, key_base, ps, keys_out, vals_out, offs,
+                                           ctl);
+    };
+    if (n <= kSmallThreads) go(small_depth_sort_kernel<1>);
+    else if (n <= 2 * kSmallThreads) go(small_depth_sort_kernel<2>);
+    else if (n <= 4 * kSmallThreads) go(small_depth_sort_kernel<4>);
+    else go(small_depth_sort_kernel<kSmallKpt>);
+    return true;
+}
+
+bool small_tile_sort(const uint32_t* keys, const uint32_t* vals, const uint32_t* d_n, int64_t max_n, int n_passes,
+                     const int* shifts, const int* bits, uint32_t* vals_out, uint2* ranges, uint32_t n_tiles,
+                     uint16_t* ranks, uint32_t* clear_bits, hipStream_t s) {
+    if (max_n <= 0 || max_n > kSmallTileSort || n_tiles > kSmallSortTiles) return false;
+    const SmallPasses ps = small_passes(n_passes, shifts, bits);
+    const uint32_t words = clear_bits ? (uint32_t)record_bit_words(max_n) : 0u;
+    auto go = [&](auto kernel) {
+        kernel<<<1, kSmallThreads, 0, s>>>(keys, vals, d_n, max_n, ps, vals_out, ranges, n_tiles, ranks, clear_bits,
+                                           words);
+    };
+    if (max_n <= 4 * kSmallThreads) go(small_tile_sort_kernel<4>);
+    else if (max_n <= 8 * kSmallThreads) go(small_tile_sort_kernel<8>);
+    else go(small_tile_sort_kernel<kSmallTileKpt>);
+    return true;
+}
+
 int64_t record_bit_words(int64_t max_inst) {
     const int64_t chunk = kThreads * kTileKeysPerThread;   // the tile passes' workgroup positions
     return ((max_inst > 0 ? max_inst : 1) + chunk - 1) / chunk * (chunk / 32);

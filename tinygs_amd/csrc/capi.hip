@@ -534,19 +534,24 @@ static int rasterizer_forward(tgs_rasterizer* r, const tgs_camera* camera, void*
     int psel;
     {
         StageScope sc(ST_DEPTH, s);
-        launch_compact_visible(r->n_touched.as<uint32_t>(), r->depth_key.as<uint32_t>(), n, sp.key_base,
-                               sp.dshift[0], sp.dbits[0], pk[0], pv[0], pn[0], r->radix_counts.as<uint32_t>(),
-                               r->block_n.as<uint32_t>(), ctl, s);
+        const bool small = small_depth_sort(r->n_touched.as<uint32_t>(), r->depth_key.as<uint32_t>(), n, sp.key_base,
+                                            sp.n_dp, sp.dshift, sp.dbits, pk[0], pv[0], r->offs.as<uint32_t>(), ctl,
+                                            s);
+        if (!small)
+            launch_compact_visible(r->n_touched.as<uint32_t>(), r->depth_key.as<uint32_t>(), n, sp.key_base,
+                                   sp.dshift[0], sp.dbits[0], pk[0], pv[0], pn[0], r->radix_counts.as<uint32_t>(),
+                                   r->block_n.as<uint32_t>(), ctl, s);
         if (!nosync) {
             // V, I and the sticky error flag go to the host while the depth sort runs
             TGS_HIP(hipMemcpyAsync(r->h_counters, ctl, 3 * sizeof(uint32_t), hipMemcpyDeviceToHost, s));
             TGS_HIP(hipEventRecord(r->ev_counts, s));
         }
-        bool offs_done = false;
-        psel = radix_sort(pk, pv, pn, &ctl->V, n, true, sp.n_dp, sp.dshift, sp.dbits, r->radix_counts.as<uint32_t>(),
-                          ctl->tickets + kTicketDepth, status, &ctl->epoch_base, r->epoch, &ctl->err,
-                          r->block_n.as<uint32_t>(), r->offs.as<uint32_t>(), &offs_done, nullptr, 0u, nullptr,
-                          nullptr, nullptr, s);
+        bool offs_done = small;
+        psel = small ? 0
+                     : radix_sort(pk, pv, pn, &ctl->V, n, true, sp.n_dp, sp.dshift, sp.dbits,
+                                  r->radix_counts.as<uint32_t>(), ctl->tickets + kTicketDepth, status,
+                                  &ctl->epoch_base, r->epoch, &ctl->err, r->block_n.as<uint32_t>(),
+                                  r->offs.as<uint32_t>(), &offs_done, nullptr, 0u, nullptr, nullptr, nullptr, s);
         if (psel < 0) return fail(TGS_ERR_STATE, "depth sort digit width");
         r->depth_key_base = sp.key_base;
         if (!offs_done) launch_instance_offsets(pn[psel], n, r->offs.as<uint32_t>(), ctl, status, r->epoch, s);
@@ -587,11 +592,18 @@ static int rasterizer_forward(tgs_rasterizer* r, const tgs_camera* camera, void*
     {
         StageScope sc(ST_TILES, s);
         // fp32: the instances' ranks out of the keys' high bits, record bits cleared
-        isel = radix_sort(ik, iv, nullptr, d_inst, cap, false, sp.n_tp, sp.tshift, sp.tbits,
-                          r->radix_counts.as<uint32_t>(), ctl->tickets + kTicketTile, status, &ctl->epoch_base,
-                          r->epoch, &ctl->err, nullptr, nullptr, nullptr, r->ranges.as<uint2>(), (uint32_t)T,
-                          &ranges_done, f16 ? nullptr : r->iranks.as<uint16_t>(),
-                          f16 ? nullptr : r->rec_bits.as<uint32_t>(), s);
+        uint16_t* ranks = f16 ? nullptr : r->iranks.as<uint16_t>();
+        uint32_t* rec_bits = f16 ? nullptr : r->rec_bits.as<uint32_t>();
+        if (small_tile_sort(ik[0], iv[0], d_inst, cap, sp.n_tp, sp.tshift, sp.tbits, iv[1], r->ranges.as<uint2>(),
+                            (uint32_t)T, ranks, rec_bits, s)) {
+            isel = 1;
+            ranges_done = true;
+        } else {
+            isel = radix_sort(ik, iv, nullptr, d_inst, cap, false, sp.n_tp, sp.tshift, sp.tbits,
+                              r->radix_counts.as<uint32_t>(), ctl->tickets + kTicketTile, status, &ctl->epoch_base,
+                              r->epoch, &ctl->err, nullptr, nullptr, nullptr, r->ranges.as<uint2>(), (uint32_t)T,
+                              &ranges_done, ranks, rec_bits, s);
+        }
         if (isel < 0) return fail(TGS_ERR_STATE, "tile sort digit width");
         if (r->epoch >= kEpochStride) return fail(TGS_ERR_STATE, "look-back launches per forward exceed the epoch stride");
         if (!ranges_done) launch_tile_ranges(ik[isel], d_inst, cap, r->ranges.as<uint2>(), T, s);
