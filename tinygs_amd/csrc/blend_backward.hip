@@ -9,16 +9,15 @@
 //
 // MI355X design:
 //   * the work item is the same bucket, but the wave is pixel-parallel: lane
-//     l owns column l % 16 of the tile at rows l / 16 + 4 s, s = 0..3, so every
-//     image / gradient access of four rows is two contiguous 128-byte runs
-//     (512-byte ones for checkpoints), and a lane has one X per Gaussian: its
-//     part of sigma is formed once, and the sums weighed by X and X^2 are one
-//     multiplication each after the lane's four pixels are summed;
+//     l owns pixels l, 64 + l, 128 + l, 192 + l of the tile, i.e. one lane of
+//     each 8x8 block, so every image / gradient / checkpoint access of a
+//     block is one contiguous 256-byte (1 KiB for checkpoints) run;
 //   * the 32 records of the bucket are staged in a wave-private LDS slice and
 //     read back as three broadcast float4 per Gaussian;
-//   * per Gaussian, each lane first sums its four pixels in registers; the
-//     sums of two Gaussians are then reduced across the wave together
-//     (wave_reduce_shared), so the cross-lane work is shared by 512 pixels;
+//   * per Gaussian, each lane first sums its four pixels in registers, then
+//     the 11 sums are reduced across the wave once (gfx950
+//     v_permlane32_swap / v_permlane16_swap + DPP row butterfly), so the
+//     cross-lane work is shared by 256 pixels;
 //   * waves take items from a device-side list (built by the forward, one
 //     entry per bucket below the tile's last contributor, carrying its first
 //     instance and count) through 64 queue counters on separate cache lines,
@@ -48,15 +47,6 @@
 
 namespace tgs {
 
-// VALU issue bounds the kernel (above 90% busy): 125 instructions per Gaussian
-// and 256 pixels, of which the pixels' own terms are 76, the column and row
-// parts 8, the lane's sums 17 and the wave reduction 20. With lanes owning one
-// pixel per 8x8 block (X of two columns), every register reduced through four
-// row steps and the sigma clamp an instruction of its own it took 148:
-// 208 -> 186 us (1M Gaussians, 1920x1080), 139 -> 128 (100k, 800x800),
-// 542 -> 490 (375k, 3840x2160); with |dL/dmean2d| 254 -> 235 (500k, 1600x1060).
-// Capped at five waves per SIMD (96 registers) it is no faster. Reducing by
-// fp32 matrix instructions (113 VALU) took 240 us: their time adds to the VALU's.
 constexpr int kBwdVals = 11;
 constexpr float kLog2e = 1.4426950408889634f;
 
@@ -74,18 +64,7 @@ __global__ void __launch_bounds__(256) blend_backward_kernel(
     __shared__ float s_part[4][kBwdVals + 1][kBucket + 1];   // +1: the four row writers hit four banks
 
     const uint32_t w = threadIdx.x >> 6, lane = threadIdx.x & 63u;
-    const uint32_t col = lane & 15u, row = lane >> 4;   // tile column and first row of this lane's pixels
-    // where a pair's reduced values go: value i is value i % kVals of Gaussian
-    // k + i / kVals, entry (i % kVals, k + i / kVals) of s_part[w]
-    constexpr int kVals = ABS ? kBwdVals : kBwdVals - 2;
-    constexpr int kRegs = (2 * kVals + 3) / 4;
-    const int i_lo = 4 * (int)reduce_slot(lane) + row_value(row);
-    const int i_hi = 16 + (kRegs == 6 && (lane & 8u) ? 4 : 0) + row_value(row);
-    float* const part = &s_part[w][0][0];
-    constexpr int kPartRow = kBucket + 1;
-    const int at_lo = (i_lo % kVals) * kPartRow + i_lo / kVals, at_hi = (i_hi % kVals) * kPartRow + i_hi / kVals;
-    const bool put_lo = (lane & 3u) == 0u;
-    const bool put_hi = (kRegs == 6 ? (lane & 7u) == 0u : (lane & 15u) == 0u) && i_hi < 2 * kVals;
+    const int q0 = row_value(lane >> 4);   // first value index this lane's row holds after wave_reduce12
     const uint32_t n_items = ctl->n_items;
     const uint32_t cs = cam.tiled_w * cam.tiled_h * 64u;
     // this wave's queue (its items: bwd_queue_item); its counter has a cache line to itself
@@ -125,12 +104,12 @@ __global__ void __launch_bounds__(256) blend_backward_kernel(
             s_part[w][kBwdVals][lane] = u2f(mask);
         }
 
-        // ---- per-pixel state at the bucket start
+        // ---- per-pixel state at the bucket start. Pixel s of this lane sits
+        // at column x[s & 1], row y[s >> 1] (two columns and two rows 8 apart)
         const uint32_t gx = tile % cam.grid_w, gy = tile / cam.grid_w;
         const uint32_t slot0 = (first - (uint32_t)j0) / (uint32_t)kBucket + tile;   // tile's first checkpoint slot
-        const uint32_t px = gx * 16u + col;
-        const float pcx = (float)px + 0.5f;
-        float pcy[4];
+        const float pcx0 = (float)(gx * 16u + (lane & 7u)) + 0.5f, pcx1 = pcx0 + 8.0f;
+        const float pcy0 = (float)(gy * 16u + (lane >> 3)) + 0.5f, pcy1 = pcy0 + 8.0f;
         float g0[4], g1[4], g2[4], Tb[4], AG[4];
         int32_t lk[4];
         uint32_t pix[4];
@@ -140,23 +119,21 @@ __global__ void __launch_bounds__(256) blend_backward_kernel(
         // an existing bucket is always allocated, whatever the pixel)
 #pragma unroll
         for (int s = 0; s < 4; ++s) {
-            const uint32_t py = gy * 16u + 4u * (uint32_t)s + row;
-            pcy[s] = (float)py + 0.5f;
+            const uint32_t px = gx * 16u + (uint32_t)(s & 1) * 8u + (lane & 7u);
+            const uint32_t py = gy * 16u + (uint32_t)(s >> 1) * 8u + (lane >> 3);
             in[s] = px < cam.width && py < cam.height;
             // outside pixels read element 0 (always allocated) and are masked below
             pix[s] = in[s] ? tiled_index(py, px, cam.tiled_w) : 0u;
             lk[s] = (int32_t)n_contrib[pix[s]] - j0;
         }
-        // in-tile index (8x8 blocks) of the lane's first pixel; its other rows follow at 32, 128 and 160
-        const size_t ck_base = (size_t)(b > 0 ? slot0 + b - 1u : 0u) * kTilePixels + (col >> 3) * 64u + row * 8u +
-                               (col & 7u);
+        const size_t ck_base = (size_t)(b > 0 ? slot0 + b - 1u : 0u) * kTilePixels + lane;
         int32_t kmax = 0;
 #pragma unroll
         for (int s = 0; s < 4; ++s) {
             const uint32_t pi = pix[s];
             const float i0 = image[pi], i1 = image[pi + cs], i2 = image[pi + 2 * cs];
             const float q0v = grad_image[pi], q1v = grad_image[pi + cs], q2v = grad_image[pi + 2 * cs];
-            float4 ck = ckpt[ck_base + (uint32_t)(s >> 1) * 128u + (uint32_t)(s & 1) * 32u];
+            float4 ck = ckpt[ck_base + (uint32_t)s * 64u];
             if (b == 0) ck = make_float4(0.f, 0.f, 0.f, 1.f);
             const bool act = in[s] && lk[s] > 0;
             lk[s] = act ? lk[s] : 0;
@@ -179,8 +156,7 @@ __global__ void __launch_bounds__(256) blend_backward_kernel(
         wave_lds_sync();
 
         // Gaussian k of the bucket: updates the pixels' state and leaves the
-        // lane's sums in acc: colours, pp, pp X^2, pp X Y, pp Y^2, pp X, pp Y
-        // (ABS: then the |dL/dmean2d| sums)
+        // wave's per-lane sums in acc[0..8] (and the |dL/dmean2d| sums in 9, 10)
         auto gaussian = [&](int32_t k, float* acc) {
             const float4 r0 = s_rec[w][0][k];   // mx, my, a/2 L, b L
             const float4 r1 = s_rec[w][1][k];   // c/2 L, opacity, a, c
@@ -192,68 +168,93 @@ __global__ void __launch_bounds__(256) blend_backward_kernel(
                     AG[s] = lk[s] == k ? 0.f : AG[s];
                 }
             }
-            // sigma' = (A X) X + Y (b X + C Y), its X parts formed once
-            const float X = r0.x - pcx;
-            const float AXX = (r0.z * X) * X, BX = r0.w * X;
-            float sp = 0.f, sy = 0.f, syy = 0.f;
+            // offsets of the two columns and rows; sigma' = X (A X + B Y) + C Y^2
+            // with its X and Y^2 parts formed once per column / row
+            const float X[2] = {r0.x - pcx0, r0.x - pcx1}, Y[2] = {r0.y - pcy0, r0.y - pcy1};
+            const float AX[2] = {r0.z * X[0], r0.z * X[1]};
+            const float CYY[2] = {(r1.x * Y[0]) * Y[0], (r1.x * Y[1]) * Y[1]};
+            acc[11] = 0.f;
+            if constexpr (!ABS) acc[9] = acc[10] = 0.f;
+            float pp[4];
 #pragma unroll
             for (int s = 0; s < 4; ++s) {
-                const float Y = r0.y - pcy[s];
-                const float sg = __builtin_fmaf(Y, __builtin_fmaf(r1.x, Y, BX), AXX);
-                // exp(-max(sigma, 0)): the clamp to [0, 1] is a modifier of the exponential
-                const float G = __builtin_amdgcn_fmed3f(__builtin_amdgcn_exp2f(-sg), 0.f, 1.f);
+                const int xi = s & 1, yi = s >> 1;
+                const float sg = __builtin_fmaf(X[xi], __builtin_fmaf(r0.w, Y[yi], AX[xi]), CYY[yi]);
+                const float G = __builtin_amdgcn_exp2f(-__builtin_fmaxf(sg, 0.f));
                 const float ab = __builtin_fminf(r1.y * G, kMaxAlpha);
                 const float wgt = Tb[s] * ab;
                 const float cg = __builtin_fmaf(r2.z, g2[s], __builtin_fmaf(r2.y, g1[s], r2.x * g0[s]));
                 AG[s] = __builtin_fmaf(-wgt, cg, AG[s]);
                 const float oma = 1.0f - ab;
                 const float dalpha = __builtin_fmaf(Tb[s], cg, -(AG[s] * __builtin_amdgcn_rcpf(oma)));
-                const float pp = ab * dalpha, ppy = pp * Y;
-                // pixel 0 starts each sum (no add of a zero)
+                pp[s] = ab * dalpha;
+                // colour sums; pixel 0 starts each (no add of a zero)
                 acc[0] = s == 0 ? wgt * g0[s] : __builtin_fmaf(wgt, g0[s], acc[0]);
                 acc[1] = s == 0 ? wgt * g1[s] : __builtin_fmaf(wgt, g1[s], acc[1]);
                 acc[2] = s == 0 ? wgt * g2[s] : __builtin_fmaf(wgt, g2[s], acc[2]);
-                sp = s == 0 ? pp : sp + pp;
-                sy = s == 0 ? ppy : sy + ppy;
-                syy = s == 0 ? ppy * Y : __builtin_fmaf(ppy, Y, syy);
                 if constexpr (ABS) {   // |dL/dmean2d| needs each pixel's own value
-                    const float hp = pp * X;
-                    const float gmx = __builtin_fmaf(hp, r1.z, ppy * r2.w);
-                    const float gmy = __builtin_fmaf(hp, r2.w, ppy * r1.w);
+                    const float hp = pp[s] * X[xi], hq = pp[s] * Y[yi];
+                    const float gmx = __builtin_fmaf(hp, r1.z, hq * r2.w);
+                    const float gmy = __builtin_fmaf(hp, r2.w, hq * r1.w);
                     acc[9] = s == 0 ? __builtin_fabsf(gmx) : acc[9] + __builtin_fabsf(gmx);
                     acc[10] = s == 0 ? __builtin_fabsf(gmy) : acc[10] + __builtin_fabsf(gmy);
                 }
                 Tb[s] *= oma;
             }
-            const float sx = X * sp;
-            acc[3] = sp;
-            acc[4] = X * sx;
-            acc[5] = X * sy;
-            acc[6] = syy;
-            acc[7] = sx;
-            acc[8] = sy;
+            // sums of pp, pp X^2, pp X Y, pp Y^2, pp X, pp Y over the four pixels
+            // from the column sums (pixels 0 + 2, 1 + 3) and row sums (0 + 1, 2 + 3)
+            {
+                const float R0 = pp[0] + pp[1], R1 = pp[2] + pp[3];
+                const float C0 = pp[0] + pp[2], C1 = pp[1] + pp[3];
+                acc[3] = R0 + R1;
+                acc[4] = __builtin_fmaf(X[0] * X[0], C0, (X[1] * X[1]) * C1);
+                acc[5] = __builtin_fmaf(Y[0], __builtin_fmaf(X[0], pp[0], X[1] * pp[1]),
+                                        Y[1] * __builtin_fmaf(X[0], pp[2], X[1] * pp[3]));
+                acc[6] = __builtin_fmaf(Y[0] * Y[0], R0, (Y[1] * Y[1]) * R1);
+                acc[7] = __builtin_fmaf(X[0], C0, X[1] * C1);
+                acc[8] = __builtin_fmaf(Y[0], R0, Y[1] * R1);
+            }
         };
-        // two Gaussians per reduction; a last single one goes with zeros, whose
-        // sums land in a column that nothing reads
-        auto reduce = [&](int32_t k, const float* a0, const float* a1) {
-            float v[4 * kRegs], lo, hi;
-#pragma unroll
-            for (int q = 0; q < 4 * kRegs; ++q) v[q] = q < kVals ? a0[q] : q < 2 * kVals ? a1[q - kVals] : 0.f;
-            wave_reduce_shared<kRegs>(v, lo, hi);
-            if (put_lo) part[at_lo + k] = lo;
-            if (put_hi) part[at_hi + k] = hi;
+        auto store = [&](int32_t k, const float* t, int nt) {
+            if ((lane & 15u) == 0u)
+                for (int m = 0; m < nt; ++m)
+                    if (4 * m + q0 < kBwdVals) s_part[w][4 * m + q0][k] = t[m];
         };
         int32_t k = 0;
-        for (; k + 1 < kmax; k += 2) {
-            float a0[kBwdVals], a1[kBwdVals];
-            gaussian(k, a0);
-            gaussian(k + 1, a1);
-            reduce(k, a0, a1);
+        if constexpr (!ABS) {
+            // two Gaussians per reduction (values 9 and 10 stay the zeros written below)
+            for (; k + 1 < kmax; k += 2) {
+                float acc2[18], acc1[12];
+                gaussian(k, acc1);
+#pragma unroll
+                for (int q = 0; q < 9; ++q) acc2[q] = acc1[q];
+                gaussian(k + 1, acc1);
+#pragma unroll
+                for (int q = 0; q < 9; ++q) acc2[9 + q] = acc1[q];
+                float t[5];
+                wave_reduce18(acc2, t);
+                if ((lane & 15u) == 0u) {
+#pragma unroll
+                    for (int m = 0; m < 5; ++m) {
+                        const int i = 4 * m + q0;   // value i % 9 of Gaussian k + i / 9
+                        if (i < 18) s_part[w][i % 9][k + i / 9] = t[m];
+                    }
+                    if (q0 == 0) {
+                        s_part[w][9][k] = s_part[w][10][k] = 0.f;
+                        s_part[w][9][k + 1] = s_part[w][10][k + 1] = 0.f;
+                    }
+                }
+            }
         }
-        if (k < kmax) {
-            float a0[kBwdVals], a1[kBwdVals] = {};
-            gaussian(k, a0);
-            reduce(k, a0, a1);
+        for (; k < kmax; ++k) {
+            float acc[12];
+            gaussian(k, acc);
+            float t[3];
+            if constexpr (ABS)
+                wave_reduce12(acc, t);
+            else
+                wave_reduce9(acc, t);   // values 9-11 are zero: their swaps are skipped
+            store(k, t, 3);
         }
         wave_lds_sync();
 
@@ -261,7 +262,7 @@ __global__ void __launch_bounds__(256) blend_backward_kernel(
             const uint32_t k = lane;
             const bool ev = (int32_t)lane < kmax;   // evaluated (always true: kmax == cnt by construction)
             const uint32_t mask = f2u(s_part[w][kBwdVals][k]);
-            auto val = [&](int q) { return ev && q < kVals ? s_part[w][q][k] : 0.f; };
+            auto val = [&](int q) { return ev ? s_part[w][q][k] : 0.f; };
             // record order: mean2d(2), abs(2), conic(3), colour(3), alpha partial, 0
             float4* dst = records + 3 * (size_t)slot;
             // dL/dmean2d = conic . (sum pp X, sum pp Y), applied once per Gaussian
