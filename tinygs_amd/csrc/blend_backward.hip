@@ -14,10 +14,9 @@
 //     block is one contiguous 256-byte (1 KiB for checkpoints) run;
 //   * the 32 records of the bucket are staged in a wave-private LDS slice and
 //     read back as three broadcast float4 per Gaussian;
-//   * per Gaussian, each lane first sums its four pixels in registers, then
-//     the 11 sums are reduced across the wave once (gfx950
-//     v_permlane32_swap / v_permlane16_swap + DPP row butterfly), so the
-//     cross-lane work is shared by 256 pixels;
+//   * per Gaussian, each lane first sums its four pixels in registers; the
+//     sums of two Gaussians are then reduced across the wave together
+//     (wave_reduce_shared), so the cross-lane work is shared by 512 pixels;
 //   * waves take items from a device-side list (built by the forward, one
 //     entry per bucket below the tile's last contributor, carrying its first
 //     instance and count) through 64 queue counters on separate cache lines,
@@ -47,6 +46,16 @@
 
 namespace tgs {
 
+// VALU issue bounds the kernel (above 90% busy): about 138 instructions per
+// Gaussian and 256 pixels, of which the wave reduction is 20. Reducing every
+// register through all four row steps, storing the row sums register by
+// register and clamping sigma apart took 148: 208 -> 196 us (1M Gaussians,
+// 1920x1080), 139 -> 131 (100k, 800x800), 542 -> 506 (375k, 3840x2160); with
+// |dL/dmean2d| 254 -> 240 (500k, 1600x1060). Capped at five waves per SIMD with
+// |dL/dmean2d| it is no faster. Reducing by fp32 matrix instructions (113 VALU)
+// took 240 us: their time adds to the VALU's. One tile column per lane (125
+// VALU) took 186, but sums the pixels in another order, which needle-shaped
+// Gaussians' rotation gradients show up to 8e-3.
 constexpr int kBwdVals = 11;
 constexpr float kLog2e = 1.4426950408889634f;
 
@@ -64,7 +73,17 @@ __global__ void __launch_bounds__(256) blend_backward_kernel(
     __shared__ float s_part[4][kBwdVals + 1][kBucket + 1];   // +1: the four row writers hit four banks
 
     const uint32_t w = threadIdx.x >> 6, lane = threadIdx.x & 63u;
-    const int q0 = row_value(lane >> 4);   // first value index this lane's row holds after wave_reduce12
+    // where a pair's reduced values go: value i is value i % kVals of Gaussian
+    // k + i / kVals, entry (i % kVals, k + i / kVals) of s_part[w]
+    constexpr int kVals = ABS ? kBwdVals : kBwdVals - 2;
+    constexpr int kRegs = (2 * kVals + 3) / 4;
+    const int i_lo = 4 * (int)reduce_slot(lane) + row_value(lane >> 4);
+    const int i_hi = 16 + (kRegs == 6 && (lane & 8u) ? 4 : 0) + row_value(lane >> 4);
+    float* const part = &s_part[w][0][0];
+    constexpr int kPartRow = kBucket + 1;
+    const int at_lo = (i_lo % kVals) * kPartRow + i_lo / kVals, at_hi = (i_hi % kVals) * kPartRow + i_hi / kVals;
+    const bool put_lo = (lane & 3u) == 0u;
+    const bool put_hi = (kRegs == 6 ? (lane & 7u) == 0u : (lane & 15u) == 0u) && i_hi < 2 * kVals;
     const uint32_t n_items = ctl->n_items;
     const uint32_t cs = cam.tiled_w * cam.tiled_h * 64u;
     // this wave's queue (its items: bwd_queue_item); its counter has a cache line to itself
@@ -173,14 +192,13 @@ __global__ void __launch_bounds__(256) blend_backward_kernel(
             const float X[2] = {r0.x - pcx0, r0.x - pcx1}, Y[2] = {r0.y - pcy0, r0.y - pcy1};
             const float AX[2] = {r0.z * X[0], r0.z * X[1]};
             const float CYY[2] = {(r1.x * Y[0]) * Y[0], (r1.x * Y[1]) * Y[1]};
-            acc[11] = 0.f;
-            if constexpr (!ABS) acc[9] = acc[10] = 0.f;
             float pp[4];
 #pragma unroll
             for (int s = 0; s < 4; ++s) {
                 const int xi = s & 1, yi = s >> 1;
                 const float sg = __builtin_fmaf(X[xi], __builtin_fmaf(r0.w, Y[yi], AX[xi]), CYY[yi]);
-                const float G = __builtin_amdgcn_exp2f(-__builtin_fmaxf(sg, 0.f));
+                // exp(-max(sigma, 0)): the clamp to [0, 1] is a modifier of the exponential
+                const float G = __builtin_amdgcn_fmed3f(__builtin_amdgcn_exp2f(-sg), 0.f, 1.f);
                 const float ab = __builtin_fminf(r1.y * G, kMaxAlpha);
                 const float wgt = Tb[s] * ab;
                 const float cg = __builtin_fmaf(r2.z, g2[s], __builtin_fmaf(r2.y, g1[s], r2.x * g0[s]));
@@ -215,46 +233,27 @@ __global__ void __launch_bounds__(256) blend_backward_kernel(
                 acc[8] = __builtin_fmaf(Y[0], R0, Y[1] * R1);
             }
         };
-        auto store = [&](int32_t k, const float* t, int nt) {
-            if ((lane & 15u) == 0u)
-                for (int m = 0; m < nt; ++m)
-                    if (4 * m + q0 < kBwdVals) s_part[w][4 * m + q0][k] = t[m];
+        // two Gaussians per reduction; a last single one goes with zeros, whose
+        // sums land in a column that nothing reads
+        auto reduce = [&](int32_t k, const float* a0, const float* a1) {
+            float v[4 * kRegs], lo, hi;
+#pragma unroll
+            for (int q = 0; q < 4 * kRegs; ++q) v[q] = q < kVals ? a0[q] : q < 2 * kVals ? a1[q - kVals] : 0.f;
+            wave_reduce_shared<kRegs>(v, lo, hi);
+            if (put_lo) part[at_lo + k] = lo;
+            if (put_hi) part[at_hi + k] = hi;
         };
         int32_t k = 0;
-        if constexpr (!ABS) {
-            // two Gaussians per reduction (values 9 and 10 stay the zeros written below)
-            for (; k + 1 < kmax; k += 2) {
-                float acc2[18], acc1[12];
-                gaussian(k, acc1);
-#pragma unroll
-                for (int q = 0; q < 9; ++q) acc2[q] = acc1[q];
-                gaussian(k + 1, acc1);
-#pragma unroll
-                for (int q = 0; q < 9; ++q) acc2[9 + q] = acc1[q];
-                float t[5];
-                wave_reduce18(acc2, t);
-                if ((lane & 15u) == 0u) {
-#pragma unroll
-                    for (int m = 0; m < 5; ++m) {
-                        const int i = 4 * m + q0;   // value i % 9 of Gaussian k + i / 9
-                        if (i < 18) s_part[w][i % 9][k + i / 9] = t[m];
-                    }
-                    if (q0 == 0) {
-                        s_part[w][9][k] = s_part[w][10][k] = 0.f;
-                        s_part[w][9][k + 1] = s_part[w][10][k + 1] = 0.f;
-                    }
-                }
-            }
+        for (; k + 1 < kmax; k += 2) {
+            float a0[kBwdVals], a1[kBwdVals];
+            gaussian(k, a0);
+            gaussian(k + 1, a1);
+            reduce(k, a0, a1);
         }
-        for (; k < kmax; ++k) {
-            float acc[12];
-            gaussian(k, acc);
-            float t[3];
-            if constexpr (ABS)
-                wave_reduce12(acc, t);
-            else
-                wave_reduce9(acc, t);   // values 9-11 are zero: their swaps are skipped
-            store(k, t, 3);
+        if (k < kmax) {
+            float a0[kBwdVals], a1[kBwdVals] = {};
+            gaussian(k, a0);
+            reduce(k, a0, a1);
         }
         wave_lds_sync();
 
@@ -262,7 +261,7 @@ __global__ void __launch_bounds__(256) blend_backward_kernel(
             const uint32_t k = lane;
             const bool ev = (int32_t)lane < kmax;   // evaluated (always true: kmax == cnt by construction)
             const uint32_t mask = f2u(s_part[w][kBwdVals][k]);
-            auto val = [&](int q) { return ev ? s_part[w][q][k] : 0.f; };
+            auto val = [&](int q) { return ev && q < kVals ? s_part[w][q][k] : 0.f; };
             // record order: mean2d(2), abs(2), conic(3), colour(3), alpha partial, 0
             float4* dst = records + 3 * (size_t)slot;
             // dL/dmean2d = conic . (sum pp X, sum pp Y), applied once per Gaussian
@@ -306,7 +305,7 @@ void launch_backward_rows(const uint4* items, const uint32_t* inst_vals, const B
     backward_rows_kernel<<<1024, 256, 0, s>>>(items, inst_vals, ctl, rows);
 }
 
-static int g_blocks = 0;
+static int g_blocks[2] = {0, 0};   // workgroups of the two kernels (without and with |dL/dmean2d|)
 
 void launch_blend_backward(const CamParams& cam, const uint32_t* inst_vals, const uint16_t* inst_ranks,
                            const float2* mean2d, const float4* conic_opacity, const float4* color_pt,
@@ -316,24 +315,24 @@ void launch_blend_backward(const CamParams& cam, const uint32_t* inst_vals, cons
                            hipStream_t s) {
     const uint32_t n_tiles = cam.grid_w * cam.grid_h;
     if (n_tiles == 0) return;
-    if (g_blocks <= 0) {
+    int& blocks = g_blocks[with_abs ? 1 : 0];
+    if (blocks <= 0) {
         // persistent workgroups: exactly as many as can be resident at once
         int dev = 0, cus = 0, per_cu = 0;
         if (hipGetDevice(&dev) != hipSuccess ||
             hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0)
             cus = 256;
-        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, blend_backward_kernel<true>, 256, 0) !=
-                hipSuccess ||
-            per_cu <= 0)
+        const void* kernel = with_abs ? (const void*)blend_backward_kernel<true> : (const void*)blend_backward_kernel<false>;
+        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, 256, 0) != hipSuccess || per_cu <= 0)
             per_cu = 4;
-        g_blocks = cus * per_cu;
+        blocks = cus * per_cu;
     }
     if (with_abs)
-        blend_backward_kernel<true><<<(uint32_t)g_blocks, 256, 0, s>>>(
+        blend_backward_kernel<true><<<(uint32_t)blocks, 256, 0, s>>>(
             cam, inst_vals, inst_ranks, mean2d, conic_opacity, color_pt, image, grad_image, n_contrib, ckpt, items,
             ctl, rec_bits, rec_mask, rec_count, first_slot, records);
     else
-        blend_backward_kernel<false><<<(uint32_t)g_blocks, 256, 0, s>>>(
+        blend_backward_kernel<false><<<(uint32_t)blocks, 256, 0, s>>>(
             cam, inst_vals, inst_ranks, mean2d, conic_opacity, color_pt, image, grad_image, n_contrib, ckpt, items,
             ctl, rec_bits, rec_mask, rec_count, first_slot, records);
 }

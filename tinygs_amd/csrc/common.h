@@ -182,104 +182,82 @@ __device__ __forceinline__ void swap16(float& a, float& b) {
     b = __builtin_bit_cast(float, (uint32_t)r[1]);
 }
 
-// Transposed wave reduction of 12 per-lane values v[0..11] into 12 wave sums.
-// After the call, lane L of t[m] holds the sum of value 4m + row_value(L >> 4)
-// (every lane of a 16-lane row holds the same total).
-//   step 1: swap32 + add folds value pairs across the two 32-lane halves,
-//   step 2: swap16 + add folds the results across rows 0/1 and 2/3,
-//   step 3: row butterfly (row_ror 8, 4, 2, 1) on the three survivors.
-// 6 + 3 swaps, 9 adds and 12 DPP adds instead of 12 x 6 dependent DPP adds.
 // Value offset held by 16-lane row r after the swaps: rows 0..3 -> 0, 2, 1, 3.
 // Arithmetic on purpose: a lane-indexed constant table becomes a global
 // memory load inside the caller's loop.
 __device__ __forceinline__ int row_value(uint32_t row) { return (int)(((row & 1u) << 1) | (row >> 1)); }
-__device__ __forceinline__ void wave_reduce12(float v[12], float t[3]) {
-#pragma unroll
-    for (int k = 0; k < 6; ++k) {
-        float a = v[2 * k], b = v[2 * k + 1];
-        swap32(a, b);
-        v[k] = a + b;   // lanes 0-31: value 2k, lanes 32-63: value 2k+1 (half sums)
-    }
-#pragma unroll
-    for (int m = 0; m < 3; ++m) {
-        float a = v[2 * m], b = v[2 * m + 1];
-        swap16(a, b);
-        t[m] = a + b;   // rows: values 4m, 4m+2, 4m+1, 4m+3 (quarter sums)
-    }
-#pragma unroll
-    for (int m = 0; m < 3; ++m) t[m] += dpp_ror_f32<0x128>(t[m]);
-#pragma unroll
-    for (int m = 0; m < 3; ++m) t[m] += dpp_ror_f32<0x124>(t[m]);
-#pragma unroll
-    for (int m = 0; m < 3; ++m) t[m] += dpp_ror_f32<0x122>(t[m]);
-#pragma unroll
-    for (int m = 0; m < 3; ++m) t[m] += dpp_ror_f32<0x121>(t[m]);
+// Wave sums of 4 NR per-lane values (NR 5 or 6): value 4 m + row_value(lane >> 4)
+// ends in lo, m = reduce_slot(lane), for m < 4 (four lanes each), and in hi for
+// m = 4 (NR = 6: lanes 0-7 of a row; m = 5 in lanes 8-15).
+//   step 1: swap32 + add folds value pairs across the two 32-lane halves,
+//   step 2: swap16 + add folds the results across rows 0/1 and 2/3, leaving one
+//           register per 4 values, summed over the 16 lanes of a row next;
+//   step 3: pairs of registers share one: a DPP add whose bank mask covers half
+//           of the lanes leaves the other half to the next register's sum, so
+//           the row steps work on 5, 3, 2 and 2 registers (6, 3, 2, 2).
+// A value's sum is formed over lanes 32, 16, 8, 4, 2 and 1 apart in that order.
+// 40 (49) instructions; four row steps on every register took 48 (60).
+__device__ __forceinline__ uint32_t reduce_slot(uint32_t lane) {
+    const uint32_t bank = (lane >> 2) & 3u;
+    return ((bank & 1u) << 1) | (bank >> 1);
 }
-
-// Two Gaussians' 9 values at once (v[0..8] and v[9..17]): lane L of t[m]
-// (m < 5) holds the sum of value 4m + row_value(L >> 4) (values 18 and 19
-// are zero). 9 + 5 swaps, 14 adds and 20 DPP adds: 48 against 2 x 28.
-__device__ __forceinline__ void wave_reduce18(float v[18], float t[5]) {
+template <int NR>
+__device__ __forceinline__ void wave_reduce_shared(float (&v)[4 * NR], float& lo, float& hi) {
+    static_assert(NR == 5 || NR == 6, "two shared registers");
+    float t[6];
 #pragma unroll
-    for (int k = 0; k < 9; ++k) {
-        float a = v[2 * k], b = v[2 * k + 1];
-        swap32(a, b);
-        v[k] = a + b;   // lanes 0-31: value 2k, lanes 32-63: value 2k+1 (half sums)
-    }
-#pragma unroll
-    for (int m = 0; m < 4; ++m) {
-        float a = v[2 * m], b = v[2 * m + 1];
-        swap16(a, b);
-        t[m] = a + b;   // rows: values 4m, 4m+2, 4m+1, 4m+3 (quarter sums)
-    }
-    {
-        float a = v[8], b = 0.f;
-        swap16(a, b);
-        t[4] = a + b;   // rows: values 16, 18 (zero), 17, 19 (zero)
-    }
-#pragma unroll
-    for (int m = 0; m < 5; ++m) t[m] += dpp_ror_f32<0x128>(t[m]);
-#pragma unroll
-    for (int m = 0; m < 5; ++m) t[m] += dpp_ror_f32<0x124>(t[m]);
-#pragma unroll
-    for (int m = 0; m < 5; ++m) t[m] += dpp_ror_f32<0x122>(t[m]);
-#pragma unroll
-    for (int m = 0; m < 5; ++m) t[m] += dpp_ror_f32<0x121>(t[m]);
-}
-
-// wave_reduce12 for v[9..11] == 0 on every lane: the same layout of t, with
-// the swaps and adds that would only move zeros left out.
-__device__ __forceinline__ void wave_reduce9(float v[12], float t[3]) {
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
+    for (int k = 0; k < 2 * NR; ++k) {
         float a = v[2 * k], b = v[2 * k + 1];
         swap32(a, b);
         v[k] = a + b;
     }
-    {
-        float a = v[8], b = 0.f;
-        swap32(a, b);
-        v[4] = a + b;   // lanes 0-31: value 8, lanes 32-63: zero (value 9)
-    }
 #pragma unroll
-    for (int m = 0; m < 2; ++m) {
+    for (int m = 0; m < NR; ++m) {
         float a = v[2 * m], b = v[2 * m + 1];
         swap16(a, b);
         t[m] = a + b;
     }
-    {
-        float a = v[4], b = 0.f;
-        swap16(a, b);
-        t[2] = a + b;   // row values 8, 10, 9, 11: only value 8 is nonzero
-    }
-#pragma unroll
-    for (int m = 0; m < 3; ++m) t[m] += dpp_ror_f32<0x128>(t[m]);
-#pragma unroll
-    for (int m = 0; m < 3; ++m) t[m] += dpp_ror_f32<0x124>(t[m]);
-#pragma unroll
-    for (int m = 0; m < 3; ++m) t[m] += dpp_ror_f32<0x122>(t[m]);
-#pragma unroll
-    for (int m = 0; m < 3; ++m) t[m] += dpp_ror_f32<0x121>(t[m]);
+    // (a DPP read of a register needs two other instructions after its write:
+    // the order below and the s_nop keep that, the compiler does not look in)
+    if constexpr (NR == 5)
+        asm("s_nop 1\n\t"
+            "v_add_f32_dpp %0, %0, %0 row_ror:8 row_mask:0xf bank_mask:0x3\n\t"
+            "v_add_f32_dpp %1, %1, %1 row_ror:8 row_mask:0xf bank_mask:0x3\n\t"
+            "v_add_f32_dpp %2, %2, %2 row_ror:8 row_mask:0xf bank_mask:0xf\n\t"
+            "v_add_f32_dpp %0, %3, %3 row_ror:8 row_mask:0xf bank_mask:0xc\n\t"
+            "v_add_f32_dpp %1, %4, %4 row_ror:8 row_mask:0xf bank_mask:0xc\n\t"
+            "v_add_f32_dpp %2, %2, %2 row_ror:4 row_mask:0xf bank_mask:0xf\n\t"
+            "v_add_f32_dpp %0, %0, %0 row_shl:4 row_mask:0xf bank_mask:0x5\n\t"
+            "v_add_f32_dpp %0, %1, %1 row_shr:4 row_mask:0xf bank_mask:0xa\n\t"
+            "v_add_f32_dpp %2, %2, %2 quad_perm:[2,3,0,1] row_mask:0xf bank_mask:0xf\n\t"
+            "s_nop 0\n\t"
+            "v_add_f32_dpp %0, %0, %0 quad_perm:[2,3,0,1] row_mask:0xf bank_mask:0xf\n\t"
+            "v_add_f32_dpp %2, %2, %2 quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
+            "s_nop 0\n\t"
+            "v_add_f32_dpp %0, %0, %0 quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf"
+            : "+v"(t[0]), "+v"(t[2]), "+v"(t[4])
+            : "v"(t[1]), "v"(t[3]));
+    else
+        asm("s_nop 1\n\t"
+            "v_add_f32_dpp %0, %0, %0 row_ror:8 row_mask:0xf bank_mask:0x3\n\t"
+            "v_add_f32_dpp %1, %1, %1 row_ror:8 row_mask:0xf bank_mask:0x3\n\t"
+            "v_add_f32_dpp %2, %2, %2 row_ror:8 row_mask:0xf bank_mask:0x3\n\t"
+            "v_add_f32_dpp %0, %3, %3 row_ror:8 row_mask:0xf bank_mask:0xc\n\t"
+            "v_add_f32_dpp %1, %4, %4 row_ror:8 row_mask:0xf bank_mask:0xc\n\t"
+            "v_add_f32_dpp %2, %5, %5 row_ror:8 row_mask:0xf bank_mask:0xc\n\t"
+            "v_add_f32_dpp %0, %0, %0 row_shl:4 row_mask:0xf bank_mask:0x5\n\t"
+            "v_add_f32_dpp %0, %1, %1 row_shr:4 row_mask:0xf bank_mask:0xa\n\t"
+            "v_add_f32_dpp %2, %2, %2 row_shl:4 row_mask:0xf bank_mask:0x5\n\t"
+            "s_nop 0\n\t"
+            "v_add_f32_dpp %0, %0, %0 quad_perm:[2,3,0,1] row_mask:0xf bank_mask:0xf\n\t"
+            "v_add_f32_dpp %2, %2, %2 quad_perm:[2,3,0,1] row_mask:0xf bank_mask:0xf\n\t"
+            "s_nop 0\n\t"
+            "v_add_f32_dpp %0, %0, %0 quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
+            "v_add_f32_dpp %2, %2, %2 quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf"
+            : "+v"(t[0]), "+v"(t[2]), "+v"(t[4])
+            : "v"(t[1]), "v"(t[3]), "v"(t[5]));
+    lo = t[0];
+    hi = t[4];
 }
 
 // Exclusive scan of R striped values per thread over a workgroup of NW

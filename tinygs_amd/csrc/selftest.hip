@@ -44,14 +44,18 @@ __global__ void wave_selftest_kernel(const uint32_t* in, uint32_t* out) {
     const uint64_t m = ballot((v & 1u) != 0u);
     const uint32_t rank = mask_rank(m);
     out[128 + lane] = rank;
-    // transposed 12-value reduction: value q of lane L = in[(L + 5 q) & 63] + q
-    float vv[12], t[3];
-    for (int q = 0; q < 12; ++q) vv[q] = (float)(in[(lane + 5u * (uint32_t)q) & 63u] + (uint32_t)q);
-    wave_reduce12(vv, t);
-    if ((lane & 15u) == 0u) {
-        const uint32_t row = lane >> 4;
-        for (int m = 0; m < 3; ++m) out[192 + 4 * m + row_value((uint32_t)row)] = f2u(t[m]);
-    }
+    // shared-register reductions of 24 (out[192..215]) and 20 (out[216..235]) values:
+    // value q of lane L = in[(L + 5 q) & 63] + q
+    float v24[24], v20[20], lo, hi;
+    for (int q = 0; q < 24; ++q) v24[q] = (float)(in[(lane + 5u * (uint32_t)q) & 63u] + (uint32_t)q);
+    for (int q = 0; q < 20; ++q) v20[q] = v24[q];
+    const uint32_t at = 4u * reduce_slot(lane) + (uint32_t)row_value(lane >> 4);
+    wave_reduce_shared<6>(v24, lo, hi);
+    if ((lane & 3u) == 0u) out[192u + at] = f2u(lo);
+    if ((lane & 7u) == 0u) out[192 + 16 + (lane & 8u ? 4 : 0) + row_value(lane >> 4)] = f2u(hi);
+    wave_reduce_shared<5>(v20, lo, hi);
+    if ((lane & 3u) == 0u) out[216u + at] = f2u(lo);
+    if ((lane & 15u) == 0u) out[216 + 16 + row_value(lane >> 4)] = f2u(hi);
     if (lane == 0) {
         out[64] = sum;
         out[65] = mx;
