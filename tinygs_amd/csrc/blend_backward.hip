@@ -197,9 +197,10 @@ __global__ void __launch_bounds__(256) blend_backward_kernel(
             for (int s = 0; s < 4; ++s) {
                 const int xi = s & 1, yi = s >> 1;
                 const float sg = __builtin_fmaf(X[xi], __builtin_fmaf(r0.w, Y[yi], AX[xi]), CYY[yi]);
-                // exp(-max(sigma, 0)): the clamp to [0, 1] is a modifier of the exponential
-                const float G = __builtin_amdgcn_fmed3f(__builtin_amdgcn_exp2f(-sg), 0.f, 1.f);
-                const float ab = __builtin_fminf(r1.y * G, kMaxAlpha);
+                // min(o exp(-max(sigma, 0)), kMaxAlpha): where the exponential exceeds 1 (or sigma
+                // is NaN, which the clamp takes as 0) the value is o, one three-way minimum
+                const float ab =
+                    __builtin_fminf(__builtin_fminf(r1.y * __builtin_amdgcn_exp2f(-sg), r1.y), kMaxAlpha);
                 const float wgt = Tb[s] * ab;
                 const float cg = __builtin_fmaf(r2.z, g2[s], __builtin_fmaf(r2.y, g1[s], r2.x * g0[s]));
                 AG[s] = __builtin_fmaf(-wgt, cg, AG[s]);
