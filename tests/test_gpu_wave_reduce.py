@@ -17,3 +17,6 @@ def test_shared_reductions(hip):
     got = out.cpu().numpy().view(np.float32)
     for start, count in ((192, 24), (216, 20)):
         assert np.array_equal(got[start:start + count], np.float32(vals.sum() + 64 * np.arange(count))), start
+    # all 24 (20) values equal
+    for start, count in ((68, 24), (92, 20)):
+        assert np.array_equal(got[start:start + count], np.full(count, vals.sum(), np.float32)), start

@@ -188,7 +188,8 @@ __device__ __forceinline__ void swap16(float& a, float& b) {
 __device__ __forceinline__ int row_value(uint32_t row) { return (int)(((row & 1u) << 1) | (row >> 1)); }
 // Wave sums of 4 NR per-lane values (NR 5 or 6): value 4 m + row_value(lane >> 4)
 // ends in lo, m = reduce_slot(lane), for m < 4 (four lanes each), and in hi for
-// m = 4 (NR = 6: lanes 0-7 of a row; m = 5 in lanes 8-15).
+// m = 4 (NR = 5: every lane of a row; NR = 6: lanes 0-3, m = 5 in lanes 8-11,
+// the other lanes hold partial sums).
 //   step 1: swap32 + add folds value pairs across the two 32-lane halves,
 //   step 2: swap16 + add folds the results across rows 0/1 and 2/3, leaving one
 //           register per 4 values, summed over the 16 lanes of a row next;
@@ -218,7 +219,9 @@ __device__ __forceinline__ void wave_reduce_shared(float (&v)[4 * NR], float& lo
         t[m] = a + b;
     }
     // (a DPP read of a register needs two other instructions after its write:
-    // the order below and the s_nop keep that, the compiler does not look in)
+    // the order below and the s_nop keep that, the compiler does not look in.
+    // The outputs are written before the last input is read, hence "+&v": an
+    // input of equal value must not share an output's register)
     if constexpr (NR == 5)
         asm("s_nop 1\n\t"
             "v_add_f32_dpp %0, %0, %0 row_ror:8 row_mask:0xf bank_mask:0x3\n\t"
@@ -235,7 +238,7 @@ __device__ __forceinline__ void wave_reduce_shared(float (&v)[4 * NR], float& lo
             "v_add_f32_dpp %2, %2, %2 quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
             "s_nop 0\n\t"
             "v_add_f32_dpp %0, %0, %0 quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf"
-            : "+v"(t[0]), "+v"(t[2]), "+v"(t[4])
+            : "+&v"(t[0]), "+&v"(t[2]), "+&v"(t[4])
             : "v"(t[1]), "v"(t[3]));
     else
         asm("s_nop 1\n\t"
@@ -254,7 +257,7 @@ __device__ __forceinline__ void wave_reduce_shared(float (&v)[4 * NR], float& lo
             "s_nop 0\n\t"
             "v_add_f32_dpp %0, %0, %0 quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
             "v_add_f32_dpp %2, %2, %2 quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf"
-            : "+v"(t[0]), "+v"(t[2]), "+v"(t[4])
+            : "+&v"(t[0]), "+&v"(t[2]), "+&v"(t[4])
             : "v"(t[1]), "v"(t[3]), "v"(t[5]));
     lo = t[0];
     hi = t[4];

@@ -31,7 +31,8 @@ void launch_detmath(int op, const float* in, float* out, int64_t n, hipStream_t 
 }
 
 // One wave of 64 inputs -> out[0..63] inclusive scan, out[64] sum,
-// out[65] max, out[66] float-sum of (float)in as bits, out[67] lane id check.
+// out[65] max, out[66] float-sum of (float)in as bits, out[67] lane id check,
+// out[68..111] and out[192..235] wave reductions, out[128..191] mask ranks.
 __global__ void wave_selftest_kernel(const uint32_t* in, uint32_t* out) {
     const uint32_t lane = lane_id();
     const uint32_t v = in[lane];
@@ -56,6 +57,16 @@ __global__ void wave_selftest_kernel(const uint32_t* in, uint32_t* out) {
     wave_reduce_shared<5>(v20, lo, hi);
     if ((lane & 3u) == 0u) out[216u + at] = f2u(lo);
     if ((lane & 15u) == 0u) out[216 + 16 + row_value(lane >> 4)] = f2u(hi);
+    // the same with all values equal, which the compiler may keep in one register
+    // before the reduction: 24 sums in out[68..91], 20 in out[92..111]
+    for (int q = 0; q < 24; ++q) v24[q] = (float)v;
+    for (int q = 0; q < 20; ++q) v20[q] = (float)v;
+    wave_reduce_shared<6>(v24, lo, hi);
+    if ((lane & 3u) == 0u) out[68u + at] = f2u(lo);
+    if ((lane & 7u) == 0u) out[68 + 16 + (lane & 8u ? 4 : 0) + row_value(lane >> 4)] = f2u(hi);
+    wave_reduce_shared<5>(v20, lo, hi);
+    if ((lane & 3u) == 0u) out[92u + at] = f2u(lo);
+    if ((lane & 15u) == 0u) out[92 + 16 + row_value(lane >> 4)] = f2u(hi);
     if (lane == 0) {
         out[64] = sum;
         out[65] = mx;
