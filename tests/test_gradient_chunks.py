@@ -7,8 +7,8 @@ import pytest
 
 from tinygs_amd import _lib
 
-SIZES = [1, 63, 64, 65, 255, 256, 257, 1023, 1024, 1025, 1100, 2047, 2049, 4097, 131071, 131073, 262145, 524288, 524289, 525000,
-         1_000_003]
+SIZES = [1, 63, 64, 65, 255, 256, 257, 1023, 1024, 1025, 1100, 2047, 2049, 4097, 131071, 131073, 262144, 262145, 262209, 524288,
+         524289, 525000, 1_000_003]
 
 
 def _fn(name):
@@ -33,3 +33,13 @@ def test_chunk_lists_hold_every_chunk(n):
         held = sum(min(64, n - 64 * u) for u in mine)
         assert len(mine) <= chunk // 64
         assert c * chunk + held <= entries
+
+
+@pytest.mark.parametrize("n", [1, 100_000, 262_144, 262_145, 330_000, 524_288, 524_289, 1_000_003, 1 << 20])
+def test_chunks_are_resident_at_once(n):
+    """Up to 2^20 primitives every chunk's workgroup has a place on the chip (256 CUs of four workgroups each), in as
+    few rounds of 256 primitives as that takes."""
+    chunks = _fn("_ZN3tgs9pb_chunksEl")(n)
+    rounds = _fn("_ZN3tgs15pb_list_entriesEl")(n) // chunks // 256
+    assert chunks <= 1024
+    assert rounds == 1 or (n + 128 * rounds - 1) // (128 * rounds) > 1024

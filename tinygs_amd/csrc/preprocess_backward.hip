@@ -362,15 +362,23 @@ __device__ __forceinline__ void hs_result(const HalfSums& h, float4& gA, float4&
 // (index, min(count, kLightRecords + 1) | span << 5, first slot, mask word of
 // ranks 0..31) and heavy (index, first slot + span, first slot, mask word);
 // fp16 images (index, count, first slot, 0) in both lists.
-constexpr int kManyRounds = 4;
 // Rounds of 256 primitives per chunk. A chunk is a chain of dependent loads
-// whatever its size, so up to 2,048 chunks of 256 (2^19 primitives) more
-// workgroups in flight win; beyond that the chip is full anyway and a chunk
-// of 1,024 fills phase 3's waves better where few primitives are live. One
-// round against four: 8.6 / 28 us at 1,024 primitives, 24 / 49 at 100k,
-// 37 / 46 at 201k, 63 / 75 at 500k; at 1M (8 % live) 76 / 57.
-constexpr int64_t kOneRoundMax = 1 << 19;
-static int pb_rounds(int64_t n) { return n <= kOneRoundMax ? 1 : kManyRounds; }
+// whatever its size, so few rounds win while all chunks are resident at once:
+// 1,024 workgroups at four waves per SIMD on 256 CUs. A second set of chunks
+// starts when the first ends and costs more than another round; with four
+// rounds phase 3's waves are also fuller where few primitives are live.
+// One, two and four rounds took (us; 32 clusters at 1920x1080, 78k of 262,144
+// and 93k of 1M live, assigned rows): 28 / 34 / 47 at 100k, 45 / 44 / 57 at
+// 262,144, 59 / 54 / 71 at 330k, 79 / 66 / 66 at 524,288, 94 / 88 / 76 at 700k,
+// 120 / 108 / 98 at 1M; where fewer are live (a ball at 1600x1060, sparse):
+// 35 / 38 / 45 at 262,144 (22k live), 43 / 35 / 39 at 524,288 (17k live).
+constexpr int64_t kResidentChunks = 1024;
+constexpr int kMaxRounds = 4;
+static int pb_rounds(int64_t n) {
+    int rounds = 1;
+    while (rounds < kMaxRounds && n > kResidentChunks * 256 * rounds) rounds *= 2;
+    return rounds;
+}
 
 int64_t pb_chunks(int64_t n) {
     const int64_t chunk = 256 * (int64_t)pb_rounds(n);
@@ -957,10 +965,11 @@ static void launch_chunks(const GaussianView& g, int bases, const CamParams& cam
     };
     auto of_rounds = [&](auto half) {
         constexpr bool kHalf = decltype(half)::value;
-        if (pb_rounds(g.n) == 1)
-            launch(preprocess_backward_chunk_kernel<ShT, kPose, kHalf, 1>);
-        else
-            launch(preprocess_backward_chunk_kernel<ShT, kPose, kHalf, kManyRounds>);
+        switch (pb_rounds(g.n)) {
+            case 1: launch(preprocess_backward_chunk_kernel<ShT, kPose, kHalf, 1>); break;
+            case 2: launch(preprocess_backward_chunk_kernel<ShT, kPose, kHalf, 2>); break;
+            default: launch(preprocess_backward_chunk_kernel<ShT, kPose, kHalf, kMaxRounds>); break;
+        }
     };
     if (half_sums)
         of_rounds(std::true_type{});
