@@ -629,16 +629,27 @@ def test_adam_masked_matches_zeroed_rows(hip):
         assert np.array_equal(x.view(np.uint32), y.view(np.uint32))
 
 
-@pytest.mark.parametrize("near_far", [(0.0, 100.0), (1e-6, 3.0e38), (0.5, 0.5000001), (2.0, 1e4)])
-def test_depth_sort_key_range_variants(hip, orc, near_far):
+@pytest.mark.parametrize("n", [6000, 20000])
+@pytest.mark.parametrize("near_far", [(0.0, 100.0), (1e-6, 3.0e38), (0.5, 0.5000001), (2.0, 1e4), (4.0, 4.0001),
+                                      (4.0, 4.05), (3.0, 6.0)])
+def test_depth_sort_key_range_variants(hip, orc, near_far, n):
     """The depth sort subtracts bits(near) from the keys and sorts only the
     bits of bits(far) - bits(near) (1 to 4 passes; 4 full-width passes when
     near <= 0): the order and the images must be those of the oracle's
-    32-bit sort for every width."""
+    32-bit sort for every width, in the one-launch sort of few primitives
+    and in the passes of more."""
     import dataclasses
-    s = scenes.config2(seed=23, n=6000, width=160, height=128)
+    s = scenes.config2(seed=23, n=n, width=160, height=128)
     near, far = near_far
     cam = dataclasses.replace(s.camera, near=near, far=far)
     s2 = dataclasses.replace(s, camera=cam)
-    print(f"[depth keys] near={near} far={far}", flush=True)
-    _check_forward(s2, orc)
+    if near == 4.0:   # 8 or 17 key bits: most means into the slice between near and far
+        rng = np.random.default_rng(4)
+        w2c = s.camera.w2c
+        depth = s.means.astype(np.float64) @ w2c[2, :3] + w2c[2, 3]
+        to = np.where(rng.random(n) < 0.9, rng.uniform(near, far, n), depth)
+        s2 = dataclasses.replace(s2, means=(s.means + (to - depth)[:, None] * w2c[2, :3]).astype(np.float32))
+    print(f"[depth keys] near={near} far={far} n={n}", flush=True)
+    _, (pre, bins, fwd) = _check_forward(s2, orc)
+    if near in (4.0, 3.0):
+        assert bins["n_visible"] > n // 4
