@@ -105,3 +105,32 @@ def test_no_sync_forward_matches_waiting(hip):
         assert r.status() == 0
         images.append(ctx.fwd_output.image.data.cpu().numpy())
     assert np.array_equal(images[0], images[1]) and np.array_equal(images[0], images[2])
+
+
+def test_one_rasterizer_through_every_route(hip):
+    """Few primitives (waiting: the sort buffers sized by the counts), many, few, no-sync, and few with more instances
+    than the one-launch tile sort takes, on one rasterizer: the images of rasterizers of their own."""
+    import torch
+    from tinygs_amd.core import GPUBatchInput, GPUGaussian3d, Image, RasterizeContext
+    from tinygs_amd.rasterizer import create_rasterizer
+    few, many, wide = _scene(1200, 131, 77, 0.0), _scene(20000, 131, 77, 0.0), _scene(5000, 300, 213, 1.0)
+
+    def image(r, s, no_sync):
+        r.set_gaussians(GPUGaussian3d.from_scene(s))
+        ctx = RasterizeContext(fwd_input=GPUBatchInput.from_camera(s.camera))
+        ctx.fwd_output.image = Image.empty(s.camera.shape)
+        if no_sync:
+            r.reserve(100_000, s.camera.grid[0] * s.camera.grid[1])
+        r.forward(ctx, no_sync=no_sync)
+        torch.cuda.synchronize()
+        return ctx.fwd_output.image.data.cpu().numpy(), r.counts()
+
+    r = create_rasterizer("fastgs")
+    instances = []
+    for s, no_sync in ((few, False), (many, False), (few, False), (many, True), (few, True), (wide, False),
+                       (wide, True), (few, False)):
+        got, counts = image(r, s, no_sync)
+        ref, ref_counts = image(create_rasterizer("fastgs"), s, no_sync)
+        assert np.array_equal(got, ref) and counts == ref_counts and r.status() == 0
+        instances.append(counts[1])
+    assert min(instances) <= SORT_MAX < max(instances) <= 100_000

@@ -297,14 +297,14 @@ int64_t scan_status_entries(int64_t max_n) { return (max_n + kScanChunk - 1) / k
 
 // ---------------------------------------------------------------- radix sort (reduce-then-scan)
 
-// Wave w of a workgroup owns 64 * KPT consecutive keys: round r, lane l is
-// key blk + w * 64 * KPT + r * 64 + l. Digit ranks come from ballot matching
-// against a wave-private LDS histogram (a wave's LDS operations complete in
-// issue order, so rounds need no barrier).
 // Bits of the widest digit of a kernel for up to maxb digits.
 constexpr int digit_bits(int maxb) { return maxb <= 1 ? 0 : 1 + digit_bits(maxb / 2); }
 static_assert(digit_bits(kDepthMaxDigits) == 9 && digit_bits(kTileMaxDigits) == 8, "whole digits");
 
+// Wave w of a workgroup owns 64 * KPT consecutive keys: round r, lane l is
+// key blk + w * 64 * KPT + r * 64 + l. Digit ranks come from ballot matching
+// against a wave-private LDS histogram (a wave's LDS operations complete in
+// issue order, so rounds need no barrier).
 template <int KPT, int MAXB>
 __device__ __forceinline__ void rank_keys(const uint32_t key[KPT], int64_t base, int64_t n, int shift, int bits,
                                           uint32_t (*s_cnt)[MAXB], uint32_t pos[KPT]) {
@@ -684,14 +684,14 @@ int radix_sort(uint32_t* keys[2], uint32_t* vals[2], uint32_t* v2[2], const uint
 // kSmallSort primitives, or kSmallTileSort instances, one workgroup of 16 waves
 // holds everything in LDS and runs all passes itself; keys stay in registers
 // between a pass's ranking and its scatter, so a pass is a few LDS round trips.
-// Renders through these sorts against the many-launch ones: 64 against 90 us
-// (1000 primitives, 1012 instances), 88 against 102 (6000, 10418), and at the
-// limits 92 (8192, 15290) against 102 (8193, 15294). Above, one workgroup's LDS
-// and ranking time no longer pay.
+// Waiting half-image forwards, one after another, through these sorts against
+// the many-launch ones: 58 against 88 us (1000 primitives, 1732 instances), 83
+// against 101 (6000, 10,416), and at the limits 91 (8192, 14,168) against 107
+// (8193, 14,170). Above, one workgroup's LDS and ranking time no longer pay.
 constexpr int kSmallWaves = 16;
 constexpr int kSmallThreads = 64 * kSmallWaves;
 constexpr int kSmallKpt = 8, kSmallTileKpt = 16;   // largest keys per thread
-constexpr int64_t kSmallSort = kSmallThreads * kSmallKpt;
+static_assert(kSmallSort == kSmallThreads * kSmallKpt, "the largest primitive count");
 constexpr int64_t kSmallTileSort = kSmallThreads * kSmallTileKpt;
 // one workgroup also initialises the tile ranges: 64 KB of them at most
 constexpr uint32_t kSmallSortTiles = 8192;
@@ -884,10 +884,48 @@ static SmallPasses small_passes(int n_passes, const int* shifts, const int* bits
     return ps;
 }
 
-bool small_depth_sort(const uint32_t* n_touched, const uint32_t* depth_key, int64_t n, uint32_t key_base,
-                      int n_passes, const int* shifts, const int* bits, uint32_t* keys_out, uint32_t* vals_out,
-                      uint32_t* offs, BinCtl* ctl, hipStream_t s) {
-    if (n <= 0 || n > kSmallSort) return false;
+// V and I ahead of the sort: a waiting forward's host reads them, sizes the
+// instance buffers and queues the rest while the sort runs. Left to the sort
+// alone they came after it: forwards of 6000 primitives (10,416 instances, half
+// images) took 88 us one after another and a new rasterizer's first 169, now 83
+// and 138; of 1000 (1732 instances) 63 and 125, now 58 and 114.
+__global__ void __launch_bounds__(kSmallThreads) small_counts_kernel(const uint32_t* __restrict__ n_touched, uint32_t n,
+                                                                     BinCtl* __restrict__ ctl) {
+    __shared__ uint32_t s_v[kSmallWaves], s_i[kSmallWaves];
+    const uint32_t t = threadIdx.x;
+    uint32_t v = 0, inst = 0;
+#pragma unroll
+    for (int r = 0; r < kSmallKpt; ++r) {
+        const uint32_t i = t + (uint32_t)(kSmallThreads * r);
+        const uint32_t nt = i < n ? n_touched[i] : 0u;
+        v += nt > 0u ? 1u : 0u;
+        inst += nt;
+    }
+    v = wave_sum_u32(v);
+    inst = wave_sum_u32(inst);
+    if ((t & 63u) == 0u) {
+        s_v[t >> 6] = v;
+        s_i[t >> 6] = inst;
+    }
+    __syncthreads();
+    if (t == 0) {
+        v = inst = 0;
+        for (int k = 0; k < kSmallWaves; ++k) {
+            v += s_v[k];
+            inst += s_i[k];
+        }
+        ctl->V = v;
+        ctl->I = inst;
+    }
+}
+
+void launch_small_counts(const uint32_t* n_touched, int64_t n, BinCtl* ctl, hipStream_t s) {
+    small_counts_kernel<<<1, kSmallThreads, 0, s>>>(n_touched, (uint32_t)n, ctl);
+}
+
+void launch_small_depth_sort(const uint32_t* n_touched, const uint32_t* depth_key, int64_t n, uint32_t key_base,
+                             int n_passes, const int* shifts, const int* bits, uint32_t* keys_out, uint32_t* vals_out,
+                             uint32_t* offs, BinCtl* ctl, hipStream_t s) {
     const SmallPasses ps = small_passes(n_passes, shifts, bits);
     auto go = [&](auto kernel) {
         kernel<<<1, kSmallThreads, 0, s>>>(n_touched, depth_key, (uint32_t)n, key_base, ps, keys_out, vals_out, offs,
@@ -897,7 +935,6 @@ bool small_depth_sort(const uint32_t* n_touched, const uint32_t* depth_key, int6
     else if (n <= 2 * kSmallThreads) go(small_depth_sort_kernel<2>);
     else if (n <= 4 * kSmallThreads) go(small_depth_sort_kernel<4>);
     else go(small_depth_sort_kernel<kSmallKpt>);
-    return true;
 }
 
 bool small_tile_sort(const uint32_t* keys, const uint32_t* vals, const uint32_t* d_n, int64_t max_n, int n_passes,

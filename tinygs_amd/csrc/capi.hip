@@ -503,10 +503,16 @@ static int rasterizer_forward(tgs_rasterizer* r, const tgs_camera* camera, void*
     TGS_TRY(ensure(r->n_contrib, 4 * cs, s));
     // without a host wait the instance buffers are sized by the reserved capacity up front
     const int64_t cap0 = nosync ? r->inst_cap : 0;
-    TGS_TRY(ensure(r->radix_counts, 4 * (size_t)std::max(radix_count_entries(nn, true),
-                                                          radix_count_entries(cap0 > 0 ? cap0 : 1, false)), s));
-    TGS_TRY(ensure_status(r, std::max({scan_status_entries(nn), scan_status_entries(radix_count_entries(nn, true)),
-                                       scan_status_entries(radix_count_entries(cap0 > 0 ? cap0 : 1, false))}), s));
+    // (the one-launch depth sort uses neither: a waiting forward through it sizes
+    // them once, by the instance count below, instead of growing them then, which
+    // frees the old ones and so waits for the sort)
+    const bool small = n > 0 && n <= kSmallSort;
+    if (nosync || !small) {
+        TGS_TRY(ensure(r->radix_counts, 4 * (size_t)std::max(radix_count_entries(nn, true),
+                                                              radix_count_entries(cap0 > 0 ? cap0 : 1, false)), s));
+        TGS_TRY(ensure_status(r, std::max({scan_status_entries(nn), scan_status_entries(radix_count_entries(nn, true)),
+                                           scan_status_entries(radix_count_entries(cap0 > 0 ? cap0 : 1, false))}), s));
+    }
     if (nosync) TGS_TRY(ensure_instances(r, cap0, T, s));
 
     GaussianView gv = view_of(r->g);
@@ -534,17 +540,24 @@ static int rasterizer_forward(tgs_rasterizer* r, const tgs_camera* camera, void*
     int psel;
     {
         StageScope sc(ST_DEPTH, s);
-        const bool small = small_depth_sort(r->n_touched.as<uint32_t>(), r->depth_key.as<uint32_t>(), n, sp.key_base,
-                                            sp.n_dp, sp.dshift, sp.dbits, pk[0], pv[0], r->offs.as<uint32_t>(), ctl,
-                                            s);
-        if (!small)
+        // V, I and the sticky error flag go to the host while the depth sort runs
+        auto copy_counts = [&]() -> int {
+            TGS_HIP(hipMemcpyAsync(r->h_counters, ctl, 3 * sizeof(uint32_t), hipMemcpyDeviceToHost, s));
+            TGS_HIP(hipEventRecord(r->ev_counts, s));
+            return TGS_OK;
+        };
+        if (small) {
+            if (!nosync) {
+                launch_small_counts(r->n_touched.as<uint32_t>(), n, ctl, s);
+                TGS_TRY(copy_counts());
+            }
+            launch_small_depth_sort(r->n_touched.as<uint32_t>(), r->depth_key.as<uint32_t>(), n, sp.key_base, sp.n_dp,
+                                    sp.dshift, sp.dbits, pk[0], pv[0], r->offs.as<uint32_t>(), ctl, s);
+        } else {
             launch_compact_visible(r->n_touched.as<uint32_t>(), r->depth_key.as<uint32_t>(), n, sp.key_base,
                                    sp.dshift[0], sp.dbits[0], pk[0], pv[0], pn[0], r->radix_counts.as<uint32_t>(),
                                    r->block_n.as<uint32_t>(), ctl, s);
-        if (!nosync) {
-            // V, I and the sticky error flag go to the host while the depth sort runs
-            TGS_HIP(hipMemcpyAsync(r->h_counters, ctl, 3 * sizeof(uint32_t), hipMemcpyDeviceToHost, s));
-            TGS_HIP(hipEventRecord(r->ev_counts, s));
+            if (!nosync) TGS_TRY(copy_counts());
         }
         bool offs_done = small;
         psel = small ? 0

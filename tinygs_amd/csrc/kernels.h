@@ -145,12 +145,15 @@ int radix_sort(uint32_t* keys[2], uint32_t* vals[2], uint32_t* v2[2], const uint
                uint64_t* status, const uint32_t* epoch_base, uint32_t& epoch, uint32_t* err,
                const uint32_t* first_block_n, uint32_t* offs, bool* offs_done, uint2* ranges, uint32_t n_tiles,
                bool* ranges_done, uint16_t* ranks, uint32_t* clear_bits, hipStream_t s);
-// The compaction, depth sort and instance offsets of up to 8192 primitives in
-// one launch (false, and nothing done, for more or none): the visible
+// The most primitives (1 and more) of the next two.
+constexpr int64_t kSmallSort = 8192;
+// ctl->V and ctl->I, ahead of the depth sort.
+void launch_small_counts(const uint32_t* n_touched, int64_t n, BinCtl* ctl, hipStream_t s);
+// The compaction, depth sort and instance offsets in one launch: the visible
 // primitives' keys and indices in depth order, offs[0 .. V], ctl->V and ctl->I.
-bool small_depth_sort(const uint32_t* n_touched, const uint32_t* depth_key, int64_t n, uint32_t key_base,
-                      int n_passes, const int* shifts, const int* bits, uint32_t* keys_out, uint32_t* vals_out,
-                      uint32_t* offs, BinCtl* ctl, hipStream_t s);
+void launch_small_depth_sort(const uint32_t* n_touched, const uint32_t* depth_key, int64_t n, uint32_t key_base,
+                             int n_passes, const int* shifts, const int* bits, uint32_t* keys_out, uint32_t* vals_out,
+                             uint32_t* offs, BinCtl* ctl, hipStream_t s);
 // The tile sort of up to 16384 instances over up to 8192 tiles in one launch
 // (false, and nothing done, beyond): what radix_sort leaves with ranges.
 bool small_tile_sort(const uint32_t* keys, const uint32_t* vals, const uint32_t* d_n, int64_t max_n, int n_passes,
