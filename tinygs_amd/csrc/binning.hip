@@ -961,7 +961,7 @@ int64_t record_bit_words(int64_t max_inst) {
 // ---------------------------------------------------------------- instance emission
 
 // Thread per depth-sorted primitive: its 16-byte emission record (bounds and
-// the preprocess's outcomes for rect tiles 0..31) is gathered once, its mean,
+// the preprocess's outcomes for rects up to kBigRect) is gathered once, its mean,
 // conic and threshold only for big rects (from the blend's own per-primitive
 // arrays); its instances fill the slots [offs[k], offs[k + 1]),
 // so the instance array comes out in depth order. (The gathers are random:
@@ -1118,7 +1118,7 @@ __global__ void __launch_bounds__(256) emit_kernel(const uint32_t* __restrict__ 
         const uint32_t jp = readlane_u32(p, j), joff = readlane_u32(off, j), jend = readlane_u32(end, j);
         uint32_t done = 0;
         walk_big_rect(readlane_u32(nrect, j), readlane_u32(org, j), readlane_u32(bw, j),
-                      [&](uint32_t, bool valid, uint32_t tx, uint32_t ty) {
+                      [&](bool valid, uint32_t tx, uint32_t ty) {
                           const bool hit =
                               valid && emit_test<kHalf>(jmx, jmy, jw0, jw1, jw2, jia, jic, tx, ty, jpt);
                           const uint64_t hm = ballot(hit);

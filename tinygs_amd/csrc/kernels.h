@@ -35,8 +35,8 @@ struct GradView {
 
 // ---- preprocess (kernels_forward.cuh:157-412)
 // erec[i] (emission record, 16 B, the part the instance emission always reads):
-// {x_min | x_max << 16, y_min | y_max << 16, exact-test outcome of the rect
-// tiles 0..31 (bit k: row-major rect tile k), 0}. ctl (may be null): the
+// {x_min | x_max << 16, y_min | y_max << 16, exact-test outcomes of a rect of at
+// most 32 tiles (bit k: row-major rect tile k; larger rects 0), 0}. ctl (may be null): the
 // binning control block, reset by the first workgroup (bin_ctl_reset_block).
 struct BinCtl;
 void launch_preprocess(const GaussianView& g, const CamParams& cam, uint32_t* n_touched, uint4* erec,
@@ -164,7 +164,7 @@ bool small_tile_sort(const uint32_t* keys, const uint32_t* vals, const uint32_t*
 int64_t record_bit_words(int64_t max_inst);
 // Instances in depth order: thread per depth-sorted primitive k < ctl->V,
 // slots [offs[k], offs[k + 1]).
-// Rect tiles past the first 32 take the exact tile test with mean2d[p], the
+// Rects of more than 32 tiles take the exact tile test with mean2d[p], the
 // conic words x, y, z of conic_words[p] and the power threshold in the w of
 // thr_words[p] (conic_opacity and color_pt for fp32 images, info for both
 // with FGS16).

@@ -23,8 +23,9 @@ namespace tgs {
 
 // Exact tile counts of the wave's 64 primitives: big rects one by one, the
 // others spread over the wave's lanes as one task list (rect_tasks.h). The
-// list's hits are counted, and the outcomes of rect tiles 0..31 kept as a bit
-// mask, with LDS atomics: the results do not depend on the order of the tests.
+// list's hits are counted, and its rects' outcomes kept as a bit mask (zero for
+// big rects, which the emission tests again), with LDS atomics: the results do
+// not depend on the order of the tests.
 // test(par, tile_x, tile_y) sees the owner's NP parameter words. s: this
 // wave's kRectSlice words. Called by the whole wave.
 //
@@ -72,17 +73,14 @@ __device__ __forceinline__ void wave_rect_tests(uint32_t nrect, uint32_t xmin, u
     bits = s_bits[lane];
     for (uint64_t todo = ballot(big); todo != 0ull; todo &= todo - 1ull) {
         const uint32_t j = (uint32_t)__builtin_ctzll(todo);
-        uint32_t pj[NP], c = 0, b = 0;
+        uint32_t pj[NP], c = 0;
 #pragma unroll
         for (int q = 0; q < NP; ++q) pj[q] = readlane_u32(par[q], j);
         walk_big_rect(readlane_u32(nrect, j), readlane_u32(org, j), readlane_u32(bw, j),
-                      [&](uint32_t first, bool valid, uint32_t tx, uint32_t ty) {
-                          const uint64_t hits = ballot(valid && test(pj, tx, ty));
-                          if (first == 0u) b = (uint32_t)hits;
-                          c += (uint32_t)__builtin_popcountll(hits);
+                      [&](bool valid, uint32_t tx, uint32_t ty) {
+                          c += (uint32_t)__builtin_popcountll(ballot(valid && test(pj, tx, ty)));
                       });
         cnt = lane == j ? c : cnt;
-        bits = lane == j ? b : bits;
     }
 }
 
@@ -307,8 +305,8 @@ __global__ void __launch_bounds__(256) preprocess_kernel(
     }
 
     // exact tile count over the rect (kernels_forward.cuh:87-153); the
-    // outcomes for rect tiles 0..31 (row-major in the rect) are kept as a bit
-    // mask, so the instance emission need not repeat the test there
+    // outcomes of a rect of at most kBigRect tiles (row-major) are kept as a
+    // bit mask, so the instance emission need not repeat the test there
     const float smx = m2x - 0.5f, smy = m2y - 0.5f;
     uint32_t cnt = 0, bits = 0;
     {

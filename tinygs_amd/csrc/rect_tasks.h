@@ -66,29 +66,32 @@ __device__ __forceinline__ void rect_tile_of(uint32_t k, uint32_t w, uint32_t& c
     row = q;
 }
 
-// Rects of more tiles than this are walked one by one. The emission keeps the
-// preprocess's outcomes of the first 32 tiles, so its task list then needs no
-// tile test; a walk of one step costs less than half a window of tasks, which
-// puts the break-even at about half a step, 32 tiles, as well.
+// Rects of more tiles than this are walked one by one. The emission record holds
+// the preprocess's outcomes of up to 32 tiles, so the emission's task list then
+// needs no tile test; a walk of one step costs less than half a window of tasks,
+// which puts the break-even at about half a step, 32 tiles, as well.
 constexpr uint32_t kBigRect = 32u;
 
-// Calls step(first, valid, tile x, tile y) for the tiles of one big rect, 64 per
-// step (tile first + lane); the arguments are wave-uniform. Columns and rows
-// advance by 64 / w and 64 % w, exact for any rect.
+// Calls step(valid, tile x, tile y) for the tiles of one big rect, 64 per step in
+// lane order; the arguments are wave-uniform, n > 0 (tested at the bottom of the
+// loop: 345 -> 334 us in the preprocess of 375k primitives of about 200 tiles).
+// Columns and rows advance by 64 / w and 64 % w, exact for any rect.
 template <class Step>
 __device__ __forceinline__ void walk_big_rect(uint32_t n, uint32_t org, uint32_t w, Step step) {
     uint32_t col, row, dcol, drow;
     rect_tile_of(lane_id(), w, col, row);
     rect_tile_of((uint32_t)kWave, w, dcol, drow);
-    for (uint32_t first = 0; first < n; first += (uint32_t)kWave) {
-        step(first, first + lane_id() < n, (org & 0xffffu) + col, (org >> 16) + row);
+    uint32_t first = 0;
+    do {
+        step(first + lane_id() < n, (org & 0xffffu) + col, (org >> 16) + row);
+        first += (uint32_t)kWave;
         col += dcol;
         row += drow;
         if (col >= w) {
             col -= w;
             ++row;
         }
-    }
+    } while (first < n);
 }
 
 // RN(a / b) for y = RN(1 / b), or by division where y is 0: two residual
