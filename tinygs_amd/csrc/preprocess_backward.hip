@@ -365,13 +365,15 @@ __device__ __forceinline__ void hs_result(const HalfSums& h, float4& gA, float4&
 // Rounds of 256 primitives per chunk. A chunk is a chain of dependent loads
 // whatever its size, so few rounds win while all chunks are resident at once:
 // 1,024 workgroups at four waves per SIMD on 256 CUs. A second set of chunks
-// starts when the first ends and costs more than another round; with four
-// rounds phase 3's waves are also fuller where few primitives are live.
-// One, two and four rounds took (us; 32 clusters at 1920x1080, 78k of 262,144
-// and 93k of 1M live, assigned rows): 28 / 34 / 47 at 100k, 45 / 44 / 57 at
-// 262,144, 59 / 54 / 71 at 330k, 79 / 66 / 66 at 524,288, 94 / 88 / 76 at 700k,
-// 120 / 108 / 98 at 1M; where fewer are live (a ball at 1600x1060, sparse):
-// 35 / 38 / 45 at 262,144 (22k live), 43 / 35 / 39 at 524,288 (17k live).
+// starts when the first ends and mostly costs more than another round; with
+// four rounds phase 3's waves are also fuller where few primitives are live.
+// One, two and four rounds took (us, assigned rows): 32 clusters at 1920x1080,
+// one scene over and over, 28 / 34 / 47 at 100k, 45 / 44 / 57 at 262,144,
+// 94 / 88 / 76 at 700k, 120 / 108 / 98 at 1M (93k live); three scenes in turn
+// (rows from HBM) 54 / 51 / 60 at 300k, 60 / 54 / 60 at 400k, 71 / 59 / 60 at
+// 524,288; a ball at 1600x1060 with densification info, Morton order, three in
+// turn (about 18k live, many records each) 59 / 63 / 74 at 300k, 62 / 63 / 73 at
+// 400k, 68 / 67 / 72 at 524,288.
 constexpr int64_t kResidentChunks = 1024;
 constexpr int kMaxRounds = 4;
 static int pb_rounds(int64_t n) {
